@@ -106,38 +106,25 @@ TUV_TRAFFIC_PER_POINT = 254
 
 MLP_FLOP_PER_CELL = 3 * 2 * (68 * 256 + 3 * 256 * 256 + 256 * 47)
 BF16_PEAK_TFLOPS = 2500.0
-# HBM traffic measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (scaled by
-# the counters' reading of a 1 GiB device copy: x2.0 and x1.0) on this
-# workload, profiles/rodas3_hbm_traffic_pmc.md (RODAS3) and
-# profiles/ros2_kernel_stats_and_traffic.md (ROS2).  Per cell-attempt (read +
-# written bytes), the same in every launch of a kernel: the spill traffic of
-# the per-lane LU and stage vectors, which depends on the register budget
-# (waves per SIMD).  The fused MLP: bytes per cell of one launch.  A kernel
-# without a measurement reports traffic null.
-BYTES_PER_CELL_ATTEMPT = {
-    "rodas3_blocks<64,false,false,4>": 49000 + 14200,
-    "rodas3_blocks<64,false,false,2>": 39200 + 10800,
-    "rodas3_blocks<64,false,false,1>": 29700 + 8300,
-    "rodas3_blocks<64,false,true,2>": 39000 + 11100,
-    "rodas3_blocks<64,false,true,1>": 29300 + 8500,
-    "ros2_blocks<64,4>": 31300 + 9350,          # profiles/ros2_kernel_stats_and_traffic.md
-}
-# the same for the lean library of another mechanism, by (mechanism, kernel):
-# profiles/other_mechanisms_solvers.md
-BYTES_PER_CELL_ATTEMPT_MECH = {
-    ("RELACS_MX", "rodas3_blocks<64,false,false,1>"): 29900 + 8400,
-    ("RELACS_MX", "rodas3_blocks<64,false,false,4>"): 49100 + 14100,
-    ("CB07_TUV", "rodas3_blocks<64,false,false,1>"): 17300 + 5000,
-    ("CB07_TUV", "rodas3_blocks<64,false,false,4>"): 30800 + 9700,
-    ("RACM_TUV", "rodas3_blocks<64,false,false,1>"): 78700 + 19000,
-    ("RACM_TUV", "rodas3_blocks<64,false,false,4>"): 111700 + 31300,
-}
+# HBM traffic of a block kernel per cell-attempt, measured with rocprofv3
+# --pmc FETCH_SIZE / WRITE_SIZE (scaled by the counters' reading of a 1 GiB
+# device copy), read + written; kernels without a measurement report null
+BYTES_PER_CELL_ATTEMPT = {}
 MLP_BYTES_PER_CELL = 1825
-FORM_WPS = {3: 1, 4: 2, 5: 4}
 
 
-def spill_traffic(kernel, cell_attempts):
-    b = BYTES_PER_CELL_ATTEMPT.get(kernel)
+def block_kernel(solver="rodas3"):
+    """Name of the kernel that runs the blocks of at most 64 cells."""
+    from brams_amd.mechanism import default_name
+    if default_name() == "racm_tuv":                    # one lane to a cell
+        return ("ros2_blocks<64,%d>" if solver == "ros2" else "rodas3_blocks<64,false,%d>") % 4
+    return "coop_blocks<%d,false,false>" % (1 if solver == "ros2" else 0)
+
+
+def block_traffic(kernel, cell_attempts):
+    """HBM bytes of a launch, where the kernel's bytes per attempt are measured."""
+    from brams_amd.mechanism import default_name
+    b = BYTES_PER_CELL_ATTEMPT.get((default_name(), kernel))
     return None if b is None else b * cell_attempts
 
 
@@ -361,11 +348,7 @@ def bench_plain(args, solver="ros2"):
         att_main += st.cell_attempts * share
         log("%s step %d: %.1f ms (main kernel %.1f ms, %d cell-attempts)"
             % (solver, t, st.kernel_ms, st.main_ms, st.cell_attempts))
-    lean = mech.name != "RELACS_TUV"        # a lean library (traffic measured where listed above)
-    if solver == "ros2":
-        kernel = "ros2_blocks<64,%d>" % FORM_WPS.get(abi.stats().kernel_form, 0)   # the autotuned form
-    else:
-        kernel = "rodas3_blocks<64,false,false,%d>" % FORM_WPS.get(abi.tuning()[0], 0)
+    kernel = block_kernel(solver)
     achieved = flops_main / (main_ms * 1e-3) / 1e12
     line = {
         "metric": "chem cell-steps/s, FP64 %s (CHEMISTRY=%d) warm rollout" % (uname, 3 if solver == "ros2" else 4),
@@ -382,10 +365,7 @@ def bench_plain(args, solver="ros2"):
                    "flop_model_" + solver: {"per_cell_call": f_call, "per_substep": f_sub, "per_attempt": f_att}},
         "roofline": {"bound": "fp64", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS,
-                     # spill traffic per cell-attempt, where it was measured
-                     "traffic": (BYTES_PER_CELL_ATTEMPT_MECH.get((mech.name, kernel)) * att_main / K
-                                 if (mech.name, kernel) in BYTES_PER_CELL_ATTEMPT_MECH
-                                 else None if lean else spill_traffic(kernel, att_main / K)),
+                     "traffic": block_traffic(kernel, att_main / K),
                      "kernel": kernel, "avg_ms": main_ms / K,
                      "algorithmic_bytes": (2 * mech.nspecies * 4 + 4 * 4 + mech.nr_photo * 8) * grid.ncell},
     }
@@ -631,15 +611,12 @@ def main():
         torch.cuda.synchronize()
         st = abi.stats()
         if t == 0:
-            # the first call of a grid also times the kernel forms (autotuner):
-            # the cold step's rate is taken over its own kernels' event time
-            form, tune_ms = abi.tuning()
-            cold = {"kernel_ms": st.kernel_ms, "call_ms_with_autotune": 1e3 * (time.perf_counter() - t0),
+            # the cold step's rate is taken over its kernels' event time (the
+            # first call of a grid also sets up the library's buffers)
+            cold = {"kernel_ms": st.kernel_ms, "call_ms": 1e3 * (time.perf_counter() - t0),
                     "attempts_per_cell": st.cell_attempts / st.cells,
                     "substeps_per_cell": st.cell_substeps / st.cells,
-                    "cell_steps_per_s": grid.ncell / (st.kernel_ms * 1e-3),
-                    "autotune": {"form": form, "kernel": "rodas3_blocks<64,false,false,%d>" % FORM_WPS.get(form, 0),
-                                 "ms_per_form": {"wps%d" % FORM_WPS[f]: float(tune_ms[f]) for f in FORM_WPS}}}
+                    "cell_steps_per_s": grid.ncell / (st.kernel_ms * 1e-3)}
         valid &= trusted_cells(wl["block_end"], dev) & physical_cells(ref, fbuf)
         log("spin-up step %d: %.1f ms (%d cell-attempts)" % (t, st.kernel_ms, st.cell_attempts))
         if t == 0:
@@ -709,10 +686,10 @@ def main():
             block_spread("last fp64 step")
     fp64_value = grid.ncell * K / wall_b
 
-    pk = "rodas3_blocks<64,false,false,%d>" % FORM_WPS.get(abi.stats().kernel_form, 0)
+    pk = block_kernel()
     plain = {"kernel": pk, "bound": "fp64", "unit": "TFLOP/s",
              "avg_ms": b_main_ms / K, "achieved": b_flops_main / (b_main_ms * 1e-3) / 1e12,
-             "peak": FP64_PEAK_TFLOPS, "traffic": spill_traffic(pk, b_att_main / K),
+             "peak": FP64_PEAK_TFLOPS, "traffic": block_traffic(pk, b_att_main / K),
              "algorithmic_bytes": 528 * grid.ncell}
     plain["frac"] = plain["achieved"] / plain["peak"]
     if sur is None:
@@ -726,10 +703,10 @@ def main():
         fb_flops = sum(rodas3_flops(s.fallback_cells, s.fallback_cell_substeps, s.fallback_cell_attempts)
                        for s in sstats)
         fb_att = sum(s.fallback_cell_attempts for s in sstats)
-        fk = "rodas3_blocks<64,false,true,%d>" % sstats[-1].fallback_wps
+        fk = block_kernel()
         fallback = {"kernel": fk, "bound": "fp64", "unit": "TFLOP/s",
                     "avg_ms": fb_ms / K, "achieved": fb_flops / max(fb_ms * 1e-3, 1e-9) / 1e12,
-                    "peak": FP64_PEAK_TFLOPS, "traffic": spill_traffic(fk, fb_att / K),
+                    "peak": FP64_PEAK_TFLOPS, "traffic": block_traffic(fk, fb_att / K),
                     "algorithmic_bytes": 528 * sum(s.fallback_cells for s in sstats) / K}
         fallback["frac"] = fallback["achieved"] / fallback["peak"]
         mlp = {"kernel": "mlp_infer<256,4,8,2>", "bound": "mfma", "unit": "TFLOP/s",

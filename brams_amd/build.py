@@ -29,22 +29,28 @@ HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=" + ARCH,
 # 49) although the same source built by default matches the oracle exactly
 # in outputs and attempt counts; parity at full size is checked by the
 # 1.6M-cell tests, which report accept/reject flips separately.
+# The block kernels' wave programs are written for the registers they have:
+# hoisted out of the attempt loop, their FP64 literals and mask tests fill the
+# scalar registers and spill.
+COOP_FLAGS = ["-mllvm", "-disable-machine-licm"]
 OBJ = os.path.join(PKG, "_build")
-# translation units of libbrams_chem.so.  The per-lane RODAS3 and ROS2 kernels
-# take about two minutes of compile each, so they are spread over four units
-# (rodas3_launch*.hip, rodas3_grids.hip, ros2_launch.hip) that compile in
-# parallel; the slab kernels (two minutes) live in rodas3_slab.hip.
+# translation units of libbrams_chem.so; the block kernels are spread over four
+# of them (rodas3_launch*.hip, rodas3_grids.hip, ros2_launch.hip) that compile
+# in parallel
 HIP_UNITS = ["rodas3_launch.hip", "rodas3_launch_b.hip", "rodas3_grids.hip", "ros2_launch.hip",
-             "rodas3_slab.hip", "qssa_launch.hip", "brams_chem.hip", "surrogate.hip"]
-# the mechanisms and their libraries: RELACS_TUV with every kernel form, the
-# others lean (BRAMS_MECH_LEAN: the per-lane kernels at one wave per SIMD,
-# no slab, list or several-grid forms), since one instantiation of RACM's
-# kernel takes about three minutes to compile
+             "qssa_launch.hip", "brams_chem.hip", "surrogate.hip"]
+# the mechanisms and their libraries: RELACS_TUV with every kernel, the others
+# lean (BRAMS_MECH_LEAN: no several-grid kernels)
 DEFAULT_MECH = "relacs_tuv"
 MECHS = ["racm_tuv", "relacs_tuv", "relacs_mx", "cb07_tuv"]   # longest compile first
 _KERNEL_UNITS = {"rodas3_launch.hip", "rodas3_launch_b.hip", "rodas3_grids.hip", "ros2_launch.hip",
                  "qssa_launch.hip"}
-_KERNEL_DEPS = ["rodas3_kernel.h", "rodas3_launch.h", "mech_families.h", "mechanism.h"]
+# the mechanisms that the cooperative block kernel holds; the other one runs
+# one lane to a cell (rodas3_lane.h)
+COOP_MECHS = ["relacs_tuv", "relacs_mx", "cb07_tuv"]
+_COOP_UNITS = _KERNEL_UNITS - {"qssa_launch.hip"}
+_KERNEL_DEPS = ["rodas3_kernel.h", "rodas3_coop.h", "coop_lane.h", "rodas3_lane.h", "rodas3_launch.h", "mech_families.h",
+                "mechanism.h"]
 # parallel compiles, one per available CPU (at most 16; each needs a few GB
 # of host memory)
 HIP_JOBS = int(os.environ.get("BRAMS_HIP_JOBS", str(min(16, len(os.sched_getaffinity(0))))))
@@ -58,16 +64,15 @@ def lib_file(mech):
 def mech_flags(mech):
     if mech == DEFAULT_MECH:
         return []
+    coop = ['-DBRAMS_MECH_COOP="generated/%s_coop.h"' % mech] if mech in COOP_MECHS else []
     return ['-DBRAMS_MECH_GEN="generated/%s_gen.h"' % mech,
-            '-DBRAMS_MECH_SLAB="generated/%s_slab.h"' % mech, "-DBRAMS_MECH_LEAN"]
+            '-DBRAMS_MECH_SLAB="generated/%s_slab.h"' % mech, "-DBRAMS_MECH_LEAN"] + coop
 
 
 def unit_deps(unit, mech):
-    gen_h = ["generated/%s_gen.h" % mech]
     if unit in _KERNEL_UNITS:
-        return _KERNEL_DEPS + gen_h
-    if unit == "rodas3_slab.hip":
-        return ["rodas3_slab.h", "rodas3_slab_launch.h"] + _KERNEL_DEPS + gen_h + ["generated/%s_slab.h" % mech]
+        coop = ["generated/%s_coop.h" % mech] if mech in COOP_MECHS else []
+        return _KERNEL_DEPS + ["generated/%s_gen.h" % mech] + coop
     return None     # every header
 
 
@@ -107,7 +112,7 @@ def build_hip(force=True, mechs=None):
             stale = (force or not os.path.exists(obj)
                      or os.path.getmtime(obj) < max(os.path.getmtime(f) for f in deps + [src]))
             if stale:
-                jobs.append((src, obj, mech_flags(mech)))
+                jobs.append((src, obj, mech_flags(mech) + (COOP_FLAGS if unit in _COOP_UNITS and mech in COOP_MECHS else [])))
             objs.append(obj)
         links.append((lib_file(mech), objs))
 

@@ -22,6 +22,10 @@ import os
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
+if HERE not in sys.path:
+    sys.path.insert(0, HERE)
+import gen_coop  # noqa: E402
+
 PKG = os.path.dirname(HERE)
 MECH = "relacs_tuv"
 GEN = os.path.join(PKG, "csrc", "generated")
@@ -203,24 +207,25 @@ def main():
     w("  const double H2O = 29.0 * M * vapp / (18.0 + 11.0 * vapp);")
     w("  const double lnT = log(T);")
     w("  (void)H2O; (void)lnT;")
-    for r, rx in enumerate(m["reactions"]):
-        law = rx["rate"]
+    def rate_rhs(r):
+        law = m["reactions"][r]["rate"]
         e = rate_expr(law["family"], law["params"], r)
         post = law["post"]
-        if post:
-            kind = post[0][0]
-            if kind == "mul_M_const":
-                w("  rk[%d] = (%s) * M * %s;" % (r, e, lit(post[0][1])))
-            elif kind == "mul_M":
-                w("  rk[%d] = (%s) * M;" % (r, e))
-            elif kind == "mul_H2O":
-                w("  rk[%d] = (%s) * H2O;" % (r, e))
-            elif kind == "mul_troe":
-                w("  rk[%d] = rl_troe(T, M, %s) * (%s);" % (r, ", ".join(lit(x) for x in post[0][1:]), e))
-            else:
-                raise ValueError(kind)
-        else:
-            w("  rk[%d] = %s;" % (r, e))
+        if not post:
+            return e
+        kind = post[0][0]
+        if kind == "mul_M_const":
+            return "(%s) * M * %s" % (e, lit(post[0][1]))
+        if kind == "mul_M":
+            return "(%s) * M" % e
+        if kind == "mul_H2O":
+            return "(%s) * H2O" % e
+        if kind == "mul_troe":
+            return "rl_troe(T, M, %s) * (%s)" % (", ".join(lit(x) for x in post[0][1:]), e)
+        raise ValueError(kind)
+
+    for r in range(nr):
+        w("  rk[%d] = %s;" % (r, rate_rhs(r)))
     w("}")
     w("")
     # ---------------- rates + fun
@@ -449,12 +454,30 @@ def main():
         json.dump(flops, fh, indent=1)
     text = "\n".join(L) + "\n"
     emit_slab(m, ns, react, prod, jt, perm, F, slot, sentries, sidx, wexpr, sum_terms, jexpr, rate_expr)
+    emit_coop(m, ns, nr, react, prod, jt, perm, F, sidx, rate_rhs)
     out = os.path.join(GEN, MECH + "_gen.h")
     old = open(out).read() if os.path.exists(out) else None
     if old != text:
         with open(out, "w") as fh:
             fh.write(text)
     print("generated %s: nstruct=%d nlu=%d" % (out, len(sentries), nlu))
+
+
+def emit_coop(m, ns, nr, react, prod, jt, perm, F, sidx, rate_rhs):
+    """The cooperative block kernels' programs (gen_coop.py)."""
+    mech = gen_coop.Mech(ns, nr, react, prod, jt, perm, F, sidx)
+    place = json.load(open(os.path.join(HERE, "coop_rows.json"))).get(MECH)
+    if place is None:                    # runs one lane to a cell (rodas3_lane.h)
+        return
+    rows = place["rows"] or gen_coop.default_rows(mech, place["waves"], place["dense"])
+    plan = gen_coop.Plan(mech, place["waves"], place["dense"], rows, place["rk_regs"],
+                         gen_coop.literal_rates(m["reactions"]))
+    text = gen_coop.emit(mech, plan, m["reactions"], rate_rhs, MECH, m["name"])
+    out = os.path.join(GEN, MECH + "_coop.h")
+    old = open(out).read() if os.path.exists(out) else None
+    if old != text:
+        with open(out, "w") as fh:
+            fh.write(text)
 
 
 def slab_out():

@@ -4,11 +4,10 @@
 // (src/brams/ccatt/chem_spack_rodas3_dyndt.f90:41-131): validates the
 // arguments, keeps persistent device buffers per grid, moves host arrays
 // to HBM and back for the Fortran entry point, and launches the kernels of
-// rodas3_kernel.h:
+// rodas3_coop.h (a workgroup to a block):
 //   1. block 1 alone (its value-based sparsity mask changes every attempt and
 //      fixes the mask for every later block, rodas3:470-506);
-//   2. the remaining blocks, 128-lane workgroups for the leading blocks with
-//      more than 64 cells and wave64 workgroups for the rest.
+//   2. the leading blocks with more than 64 cells, then the rest.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -24,7 +23,6 @@
 #include "../../include/brams_surrogate.h"
 #include "rodas3_kernel.h"
 #include "rodas3_launch.h"
-#include "rodas3_slab_launch.h"
 #include "sched_kernels.h"
 #include "jphoto_kernels.h"
 #include "sur_step_kernels.h"
@@ -71,30 +69,15 @@ struct DevBuf {
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
-// Kernel forms of the 64-cell partition blocks: the slab layouts
-// 0..kSlabVariants-1 (rodas3_slab.h) and the per-lane kernel
-// (rodas3_kernel.h) at 1, 2 and 4 waves per SIMD.  All give bit-identical
-// results; the autotuner keeps the fastest per grid.
-constexpr int kFormPerLane = brams::kSlabVariants;      // first per-lane form
-constexpr int kPerLaneWps[3] = {1, 2, 4};
-constexpr int kForms = brams::kSlabVariants + 3;
-// the per-lane forms the library holds (a lean build: 1 and 4 waves per SIMD)
+// Kernel forms of the 64-cell blocks, by the numbers that callers know
+// (brams_chem_set_form).  0..2 were layouts that never ran; 3..5 were register
+// budgets of a one-lane-per-cell kernel.  The cooperative block kernel has one
+// form, so all of 3..5 run it and there is nothing to choose.
+constexpr int kFirstForm = 3;
+constexpr int kForms = 6;
 constexpr bool form_built(int f) {
-  return f >= kFormPerLane && f < kForms && (!brams::kLeanBuild || f != kFormPerLane + 1);
+  return f >= kFirstForm && f < kForms && (!brams::kLeanBuild || f != kFirstForm + 1);
 }
-// List (fallback) launches: the per-lane kernel at 1 or 2 waves per SIMD,
-// by the launch's block count.  Measured on the 1.6M-cell rollout (ms per
-// launch, 1 / 2 waves per SIMD): 19 400 blocks 246 / 190; the 2000..6000
-// blocks of the warm steps 35.5 / 39.6 on average over 24 steps.  Timing
-// each call's choice online was too noisy to pick reliably (consecutive
-// calls differ by 10%), so the crossover is fixed.
-constexpr int kListWps[2] = {1, 2};
-constexpr int kListManyBlocks = 8192;
-// The slab forms are switched off: on gfx950 their kernels did not
-// terminate, even for a one-block grid with the attempts capped at 300,
-// while a host build of the same block integration matches the oracle bit
-// for bit.  Until that is understood every call takes the per-lane form.
-constexpr bool kSlabEnabled = false;
 
 // Device state of one grid, created on the first call for that grid and
 // kept until brams_chem_finalize (the reference allocates its block index
@@ -111,10 +94,7 @@ struct GridState {
   DevBuf cell_dt;
   std::vector<int> h_att, h_sub, h_fail, h_thresh;
   std::vector<float> h_forced;
-  int form = -1;                 // kernel form of the 64-cell blocks (-1: not tuned yet)
-  float tune_ms[kForms] = {};
-  int ros2_form = -1;            // the same for the ROS2 step (forms 3 and 5)
-  float ros2_tune_ms[kForms] = {};
+  float tune_ms[kForms] = {};    // 64-cell blocks of the grid's first RODAS3 call
   bool same(int a1, int a2, int a3, int b1, int b2, int b3, int b4) const {
     return m1 == a1 && m2 == a2 && m3 == a3 && ia == b1 && iz == b2 && ja == b3 && jz == b4;
   }
@@ -131,13 +111,8 @@ struct State {
   DevBuf sur_X, sur_out, sur_flag, sur_list, sur_chunk, sur_reason, fb_dt, fb_att, mask_all;
   // work ordering (sched_kernels.h): sort scratch and block order
   DevBuf sort_keys, sort_ids, sort_count, sort_off, order;
-  // slab kernels: per-slot scratch regions and the work-queue counter
-  DevBuf slab_lu, slab_jac, slab_rk, slab_vec, qcount;
-  long long slab_slots = 0;
-  int n_cu = 0;
-  int force_form = -1;           // brams_chem_set_form (-1: autotune per grid)
-  // autotuning scratch (copies of the state a step writes)
-  DevBuf tune_sc, tune_dt;
+  DevBuf half_y;                 // the halves of blocks of more than 64 cells
+  int force_form = -1;           // brams_chem_set_form (-1: none)
   // QSSA: count of cells that reached 1e20
   DevBuf qssa_fatal;
   // several grids in one pass: per-grid kernel parameters and work lists
@@ -177,7 +152,9 @@ constexpr size_t kNaForced = na_round(kNaFailed + sizeof(int) * kNoAllocMaxBlock
 constexpr size_t kNaThresh = na_round(kNaForced + sizeof(float) * kNoAllocMaxBlocks);      // int[max]
 constexpr size_t kNaOrderThresh = na_round(kNaThresh + sizeof(int) * kNoAllocMaxBlocks);   // int[1]
 constexpr size_t kNaCount = na_round(kNaOrderThresh + sizeof(int));                        // int[1]
-constexpr size_t kNoAllocBytes = na_round(kNaCount + sizeof(int));
+// at most 63 blocks hold more than 64 cells
+constexpr size_t kNaHalf = na_round(kNaCount + sizeof(int));
+constexpr size_t kNoAllocBytes = na_round(kNaHalf + brams::kHalfBytes * 64);
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -284,123 +261,10 @@ int order_blocks(int b0, int n, hipStream_t st) {
   return sort_desc(g.sort_keys.as<int>(), g.sort_ids.as<int>(), n, g.order.as<int>(), st);
 }
 
-// slots of a slab variant: every CU times the workgroups resident per CU
-int slab_slots(int variant, long long* nslots) {
-  const int per_cu = brams::slab_resident_per_cu(variant);
-  if (per_cu <= 0) return fail(-5, "slab kernel variant %d cannot be resident", variant);
-  *nslots = (long long)g.n_cu * per_cu;
-  return 0;
-}
-
-// per-slot scratch for n slots
-int ensure_slabs(long long n) {
-  if (n <= g.slab_slots) return 0;
-  HIP_TRY(g.slab_lu.ensure(sizeof(double) * 64 * brams::kSlabLuRows * n));
-  HIP_TRY(g.slab_jac.ensure(sizeof(double) * 64 * brams::kSlabJacRows * n));
-  HIP_TRY(g.slab_rk.ensure(sizeof(double) * 64 * brams::kSlabRkRows * n));
-  HIP_TRY(g.slab_vec.ensure(sizeof(double) * 64 * brams::kSlabVecRows * n));
-  g.slab_slots = n;
-  return 0;
-}
-
-brams::QueueParams queue(const int* order, int b0, int nitems) {
-  brams::QueueParams q{};
-  q.counter = g.qcount.as<int>();
-  q.order = order;
-  q.b0 = b0;
-  q.nitems = nitems;
-  q.lu = g.slab_lu.as<double>();
-  q.jac = g.slab_jac.as<double>();
-  q.rk = g.slab_rk.as<double>();
-  q.vec = g.slab_vec.as<double>();
-  return q;
-}
-
-// the 64-cell blocks [first64, nob) in the given kernel form; order: the
-// blocks' launch order (null: ascending)
-int launch_main(int form, const brams::StepParams& p, int first64, int nob, const int* order,
-                hipStream_t st) {
-  const int n = nob - first64;
-  if (n <= 0) return 0;
-  if (form >= kFormPerLane) {
-    brams::StepParams pm = p;
-    pm.block_order = order;
-    HIP_TRY(brams::launch_rodas3(64, false, (unsigned)n, pm, first64, st, kPerLaneWps[form - kFormPerLane]));
-    return 0;
-  }
-  long long nslots = 0;
-  int rc = slab_slots(form, &nslots);
-  if (rc) return rc;
-  nslots = std::min<long long>(nslots, n);
-  if ((rc = ensure_slabs(nslots))) return rc;
-  HIP_TRY(brams::launch_rodas3_slab(form, (unsigned)nslots, p, queue(order, first64, n), st));
-  return 0;
-}
-
-// block 1 alone: its value-based mask fixes the mask of every later block
-int launch_block1(const brams::StepParams& p, hipStream_t st) {
-  if (!kSlabEnabled || g.cur->sizes[0] > 64) {
-    HIP_TRY(brams::launch_rodas3(g.cur->sizes[0] > 64 ? 128 : 64, true, 1, p, 0, st));
-    return 0;
-  }
-  if (g.cur->sizes[0] > 64) {
-    HIP_TRY(brams::launch_rodas3(128, true, 1, p, 0, st));
-    return 0;
-  }
-  int rc = ensure_slabs(1);
-  if (rc) return rc;
-  HIP_TRY(brams::launch_rodas3_slab(brams::kSlabBlock1, 1, p, queue(nullptr, 0, 1), st));
-  return 0;
-}
-
-// Autotuner: on the first call of a grid, each kernel form (the per-lane
-// kernel at 1, 2 and 4 waves per SIMD, and the slab layouts when they are
-// switched on) integrates the call's 64-cell blocks on a scratch copy of the
-// state (block 1 has run on it first, so the mask is the call's), timed
-// with events; the fastest is kept for the grid.  The forms give
-// bit-identical results, so the choice changes speed only.  The caller's
-// arrays are not touched.
-int autotune(brams::StepParams p, int first64, int nob, hipStream_t st) {
-  GridState& gs = *g.cur;
-  const size_t nsc = sizeof(float) * MECH_NS * (size_t)p.n3d;
-  const bool to_t = (p.split == brams::kSplitParallel) && (p.ndyn == 1);
-  HIP_TRY(g.tune_sc.ensure(2 * nsc * (to_t ? 2 : 1)));
-  HIP_TRY(g.tune_dt.ensure(2 * sizeof(double) * nob));
-  float* sc0 = g.tune_sc.as<float>();
-  float* sc1 = sc0 + (size_t)MECH_NS * p.n3d;
-  float* st0 = to_t ? sc1 + (size_t)MECH_NS * p.n3d : nullptr;
-  float* st1 = to_t ? st0 + (size_t)MECH_NS * p.n3d : nullptr;
-  double* dt0 = g.tune_dt.as<double>();
-  double* dt1 = dt0 + nob;
-  HIP_TRY(hipMemcpyAsync(sc0, p.sc_p, nsc, hipMemcpyDeviceToDevice, st));
-  if (to_t) HIP_TRY(hipMemcpyAsync(st0, p.sc_t, nsc, hipMemcpyDeviceToDevice, st));
-  HIP_TRY(hipMemcpyAsync(dt0, p.last_dt, sizeof(double) * nob, hipMemcpyDeviceToDevice, st));
-  brams::StepParams q = p;
-  q.sc_p = sc0;
-  q.sc_t = st0;
-  q.last_dt = dt0;
-  int rc = launch_block1(q, st);
-  if (rc) return rc;
-  q.sc_p = sc1;
-  q.sc_t = st1;
-  q.last_dt = dt1;
-  const int f0 = kSlabEnabled ? 0 : kFormPerLane;
-  int best = f0;
-  for (int f = f0; f < kForms; ++f) {
-    if (f >= kFormPerLane && !form_built(f)) continue;
-    HIP_TRY(hipMemcpyAsync(sc1, sc0, nsc, hipMemcpyDeviceToDevice, st));
-    if (to_t) HIP_TRY(hipMemcpyAsync(st1, st0, nsc, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipMemcpyAsync(dt1, dt0, sizeof(double) * nob, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipEventRecord(g.ev0, st));
-    if ((rc = launch_main(f, q, first64, nob, nullptr, st))) return rc;
-    HIP_TRY(hipEventRecord(g.ev1, st));
-    HIP_TRY(hipEventSynchronize(g.ev1));
-    float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, g.ev0, g.ev1));
-    gs.tune_ms[f] = ms;
-    if (ms < gs.tune_ms[best]) best = f;
-  }
-  gs.form = best;
+// memory for the halves of n blocks of more than 64 cells
+int ensure_halves(int n, brams::StepParams& p) {
+  HIP_TRY(g.half_y.ensure(brams::kHalfBytes * (size_t)std::max(n, 1)));
+  p.half_y = g.half_y.as<double>();
   return 0;
 }
 
@@ -421,29 +285,25 @@ int launch_step(brams::StepParams p, hipStream_t st) {
   int nbig = 0;
   while (nbig < nob && sz[nbig] > 64) ++nbig;
   const int first64 = nbig > 1 ? nbig : 1;
-  int form = g.force_form >= 0 ? g.force_form : gs.form;
-  if (form < 0 && nob > first64) {
-    int rc = autotune(p, first64, nob, st);
-    if (rc) return rc;
-    form = gs.form;
-  }
+  const int form = g.force_form >= 0 ? g.force_form : kFirstForm;
+  int rc = ensure_halves(nbig, p);
+  if (rc) return rc;
   // the 64-cell blocks run longest first once a call on this grid has
   // counted their attempts (the order changes no block's result)
   const int* order = nullptr;
   if (nob > first64 && gs.blk_hist) {
-    int rc = order_blocks(first64, nob - first64, st);
-    if (rc) return rc;
+    if ((rc = order_blocks(first64, nob - first64, st))) return rc;
     order = g.order.as<int>();
   }
   HIP_TRY(hipEventRecord(g.ev0, st));
-  int rc = launch_block1(p, st);
-  if (rc) return rc;
+  HIP_TRY(brams::launch_rodas3_first(p, st));
   HIP_TRY(hipEventRecord(g.evb, st));
-  if (nbig > 1) HIP_TRY(brams::launch_rodas3(128, false, (unsigned)(nbig - 1), p, 1, st));
+  if (nbig > 1) HIP_TRY(brams::launch_rodas3_big((unsigned)(nbig - 1), p, 1, st));
   HIP_TRY(hipEventRecord(g.evm, st));
   g.main_cells = 0;
   if (nob > first64) {
-    if ((rc = launch_main(form, p, first64, nob, order, st))) return rc;
+    p.block_order = order;
+    HIP_TRY(brams::launch_rodas3((unsigned)(nob - first64), p, first64, st));
     for (int b = first64; b < nob; ++b) g.main_cells += sz[b];
   }
   HIP_TRY(hipEventRecord(g.ev1, st));
@@ -469,41 +329,8 @@ constexpr StructMask kStructMask = struct_mask();
 
 // The ROS2 solver (CHEMISTRY=3, chem_spack_ros_dyndt.f90) on the current
 // grid: every block alike on the full structural Jacobian, so no block-1 form
-// and no mask; the 65..127-cell blocks on 128 lanes, the 64-cell blocks
+// and no mask; the 65..127-cell blocks first, then the 64-cell blocks,
 // longest first from the second call on the grid.
-// The ROS2 step's 64-cell blocks at one and four waves per SIMD (forms 3
-// and 5, both built in every library), timed on a scratch copy of the state
-// on the first ROS2 call of a grid, as autotune() does for RODAS3; the
-// blocks are independent (no mask), so no other block runs first.
-int ros2_autotune(const brams::StepParams& p, int first64, int nob, hipStream_t st) {
-  GridState& gs = *g.cur;
-  const size_t nsc = sizeof(float) * MECH_NS * (size_t)p.n3d;
-  const bool to_t = (p.split == brams::kSplitParallel) && (p.ndyn == 1);
-  HIP_TRY(g.tune_sc.ensure(nsc * (to_t ? 2 : 1)));
-  HIP_TRY(g.tune_dt.ensure(sizeof(double) * nob));
-  brams::StepParams q = p;
-  q.sc_p = g.tune_sc.as<float>();
-  q.sc_t = to_t ? q.sc_p + (size_t)MECH_NS * p.n3d : nullptr;
-  q.last_dt = g.tune_dt.as<double>();
-  const int forms[2] = {kFormPerLane, kFormPerLane + 2};
-  int best = forms[0];
-  for (int f : forms) {
-    HIP_TRY(hipMemcpyAsync(q.sc_p, p.sc_p, nsc, hipMemcpyDeviceToDevice, st));
-    if (to_t) HIP_TRY(hipMemcpyAsync(q.sc_t, p.sc_t, nsc, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipMemcpyAsync(q.last_dt, p.last_dt, sizeof(double) * nob, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipEventRecord(g.ev0, st));
-    HIP_TRY(brams::launch_ros2(64, (unsigned)(nob - first64), q, first64, st, kPerLaneWps[f - kFormPerLane]));
-    HIP_TRY(hipEventRecord(g.ev1, st));
-    HIP_TRY(hipEventSynchronize(g.ev1));
-    float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, g.ev0, g.ev1));
-    gs.ros2_tune_ms[f] = ms;
-    if (ms < gs.ros2_tune_ms[best]) best = f;
-  }
-  gs.ros2_form = best;
-  return 0;
-}
-
 int launch_ros2_step(brams::StepParams p, hipStream_t st) {
   GridState& gs = *g.cur;
   const int nob = (int)gs.sizes.size();
@@ -519,30 +346,26 @@ int launch_ros2_step(brams::StepParams p, hipStream_t st) {
   HIP_TRY(hipMemsetAsync(gs.order_thresh.p, 0, sizeof(int), st));
   int nbig = 0;
   while (nbig < nob && gs.sizes[nbig] > 64) ++nbig;
-  // brams_chem_set_form forces the ROS2 form too (3 or 5: ROS2 has no
-  // two-wave kernel)
-  if (g.force_form == kFormPerLane + 1)
-    return fail(-6, "ROS2 has no kernel form %d (two waves per SIMD)", g.force_form);
-  if (g.force_form < 0 && gs.ros2_form < 0 && nob > nbig) {
-    int rc = ros2_autotune(p, nbig, nob, st);
-    if (rc) return rc;
-  }
-  const int form = g.force_form >= 0 ? g.force_form : gs.ros2_form;
+  // ROS2 never had a form 4
+  if (g.force_form == kFirstForm + 1)
+    return fail(-6, "ROS2 has no kernel form %d", g.force_form);
+  const int form = g.force_form >= 0 ? g.force_form : kFirstForm;
+  int rc = ensure_halves(nbig, p);
+  if (rc) return rc;
   const int* order = nullptr;
   if (nob > nbig && gs.blk_hist) {
-    int rc = order_blocks(nbig, nob - nbig, st);
-    if (rc) return rc;
+    if ((rc = order_blocks(nbig, nob - nbig, st))) return rc;
     order = g.order.as<int>();
   }
   HIP_TRY(hipEventRecord(g.ev0, st));
-  HIP_TRY(brams::launch_ros2(128, (unsigned)nbig, p, 0, st));
+  HIP_TRY(brams::launch_ros2_big((unsigned)nbig, p, 0, st));
   HIP_TRY(hipEventRecord(g.evb, st));
   HIP_TRY(hipEventRecord(g.evm, st));
   g.main_cells = 0;
   if (nob > nbig) {
     brams::StepParams pm = p;
     pm.block_order = order;
-    HIP_TRY(brams::launch_ros2(64, (unsigned)(nob - nbig), pm, nbig, st, kPerLaneWps[form - kFormPerLane]));
+    HIP_TRY(brams::launch_ros2((unsigned)(nob - nbig), pm, nbig, st));
     for (int b = nbig; b < nob; ++b) g.main_cells += gs.sizes[b];
   }
   HIP_TRY(hipEventRecord(g.ev1, st));
@@ -595,6 +418,8 @@ int collect_stats(hipStream_t st) {
   s.main_ms = ms;
   s.main_cells = g.main_cells;
   s.kernel_form = g.last_form;
+  for (int f = kFirstForm; f < kForms; ++f)
+    if (form_built(f) && gs.tune_ms[f] == 0.f) gs.tune_ms[f] = ms;
   g.stats = s;
   return (int)s.failed_blocks;
 }
@@ -653,8 +478,6 @@ int brams_chem_init(int device) {
   if (!g.evm) HIP_TRY(hipEventCreate(&g.evm));
   for (auto& e : g.sev)
     if (!e) HIP_TRY(hipEventCreate(&e));
-  g.n_cu = prop.multiProcessorCount;
-  HIP_TRY(g.qcount.ensure(sizeof(int) * 64));
   unsigned char* na = nullptr;
   if (int rc = scratch_address(&na)) return rc;
   g.init = true;
@@ -868,7 +691,7 @@ int brams_chem_rodas3_dyndt_device(const brams_chem_dev_args* a) {
 
 // The same step with no allocation: the bookkeeping sits in `scratch`, the
 // blocks run in partition order through the same kernels (block 1, then the
-// 65..127-cell blocks on 128 lanes, then the 64-cell blocks).
+// 65..127-cell blocks, then the 64-cell blocks).
 int brams_chem_rodas3_dyndt_device_noalloc(const brams_chem_dev_args* a) {
   int rc = check_device_args(a);
   if (rc) return rc;
@@ -904,10 +727,11 @@ int brams_chem_rodas3_dyndt_device_noalloc(const brams_chem_dev_args* a) {
   hipLaunchKernelGGL(brams::partition_starts, dim3((unsigned)((nob + 256) / 256)), dim3(256), 0, st, nob,
                      base, r, starts);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(brams::launch_rodas3(size0 > 64 ? 128 : 64, true, 1, p, 0, st));
-  if (nbig > 1) HIP_TRY(brams::launch_rodas3(128, false, (unsigned)(nbig - 1), p, 1, st));
+  p.half_y = reinterpret_cast<double*>(s + kNaHalf);
+  HIP_TRY(brams::launch_rodas3_first(p, st));
+  if (nbig > 1) HIP_TRY(brams::launch_rodas3_big((unsigned)(nbig - 1), p, 1, st));
   const int first64 = nbig > 1 ? nbig : 1;
-  if (nob > first64) HIP_TRY(brams::launch_rodas3(64, false, (unsigned)(nob - first64), p, first64, st));
+  if (nob > first64) HIP_TRY(brams::launch_rodas3((unsigned)(nob - first64), p, first64, st));
   hipLaunchKernelGGL(brams::count_nonzero, dim3(1), dim3(256), 0, st, p.blk_failed, nob, count);
   HIP_TRY(hipGetLastError());
   int nfail = 0;
@@ -996,6 +820,8 @@ int brams_chem_rodas3_dyndt_device_grids(const brams_chem_dev_args* a, int32_t n
              gss[y >> brams::kGridShift]->h_att[y & brams::kGridBlockMask];
     });
   hipStream_t st = (hipStream_t)a[0].stream;
+  for (brams::StepParams& p : ps)
+    if (int rc = ensure_halves((int)std::max(w1.size(), w128.size()), p)) return rc;
   const size_t nw = w1.size() + w128.size() + w64.size();
   HIP_TRY(g.multi_ps.ensure(sizeof(brams::StepParams) * ngrids));
   HIP_TRY(g.multi_work.ensure(sizeof(int) * nw));
@@ -1017,24 +843,22 @@ int brams_chem_rodas3_dyndt_device_grids(const brams_chem_dev_args* a, int32_t n
     for (int i = 0; i < ngrids; ++i) {
       const std::vector<int>& sz = gss[i]->sizes;
       while (nbig[i] < (int)sz.size() && sz[nbig[i]] > 64) ++nbig[i];
-      HIP_TRY(brams::launch_rodas3(sz[0] > 64 ? 128 : 64, true, 1, ps[i], 0, st));
+      HIP_TRY(brams::launch_rodas3_first(ps[i], st));
     }
     HIP_TRY(hipEventRecord(g.evb, st));
     for (int i = 0; i < ngrids; ++i)
-      if (nbig[i] > 1) HIP_TRY(brams::launch_rodas3(128, false, (unsigned)(nbig[i] - 1), ps[i], 1, st));
+      if (nbig[i] > 1) HIP_TRY(brams::launch_rodas3_big((unsigned)(nbig[i] - 1), ps[i], 1, st));
     HIP_TRY(hipEventRecord(g.evm, st));
     for (int i = 0; i < ngrids; ++i) {
       const int first64 = std::max(nbig[i], 1), nob = (int)gss[i]->sizes.size();
-      if (nob > first64) HIP_TRY(brams::launch_rodas3(64, false, (unsigned)(nob - first64), ps[i], first64, st, 1));
+      if (nob > first64) HIP_TRY(brams::launch_rodas3((unsigned)(nob - first64), ps[i], first64, st));
     }
   } else {
-    HIP_TRY(brams::launch_rodas3_grids(128, true, 1, (unsigned)w1.size(), dps, dw, st));
+    HIP_TRY(brams::launch_rodas3_grids(true, true, (unsigned)w1.size(), dps, dw, st));
     HIP_TRY(hipEventRecord(g.evb, st));
-    HIP_TRY(brams::launch_rodas3_grids(128, false, 1, (unsigned)w128.size(), dps, dw + w1.size(), st));
+    HIP_TRY(brams::launch_rodas3_grids(false, true, (unsigned)w128.size(), dps, dw + w1.size(), st));
     HIP_TRY(hipEventRecord(g.evm, st));
-    const int wps = w64.size() >= (size_t)brams::kRodas3ManyBlocks ? brams::kRodas3ManyWaves : 1;
-    HIP_TRY(brams::launch_rodas3_grids(64, false, wps, (unsigned)w64.size(), dps,
-                                       dw + w1.size() + w128.size(), st));
+    HIP_TRY(brams::launch_rodas3_grids(false, false, (unsigned)w64.size(), dps, dw + w1.size() + w128.size(), st));
   }
   HIP_TRY(hipEventRecord(g.ev1, st));
   // per-grid counters, then their sums (mask size: the first grid's)
@@ -1215,7 +1039,6 @@ int brams_sur_step(const brams_chem_dev_args* a, const brams_sur_model* m, brams
   //    1.6M-cell rollout (68 against 57 ms): scattered gathers cost more than
   //    the more uniform blocks save.
   long long fb_att = 0, fb_cell_att = 0, fb_cell_sub = 0, fb_failed = 0;
-  int fb_form = -1;
   if (nfb > 0) {
     const int nb = (nfb + 63) / 64;
     int* list = g.sur_list.as<int>();
@@ -1238,16 +1061,7 @@ int brams_sur_step(const brams_chem_dev_args* a, const brams_sur_model* m, brams
     q.blk_thresh = nullptr;
     q.order_thresh = nullptr;
     q.block_start = nullptr;
-    if (kSlabEnabled) {
-      long long nslots = 0;
-      if ((rc = slab_slots(brams::kSlabList, &nslots))) return rc;
-      nslots = std::min<long long>(nslots, nb);
-      if ((rc = ensure_slabs(nslots))) return rc;
-      HIP_TRY(brams::launch_rodas3_slab(brams::kSlabList, (unsigned)nslots, q, queue(nullptr, 0, nb), st));
-    } else {
-      fb_form = nb >= kListManyBlocks ? 1 : 0;
-      HIP_TRY(brams::launch_rodas3_list((unsigned)nb, q, st, kListWps[fb_form]));
-    }
+    HIP_TRY(brams::launch_rodas3((unsigned)nb, q, 0, st));
     hipLaunchKernelGGL(brams::cell_history_update, dim3((unsigned)((nfb + 255) / 256)), dim3(256), 0, st, list,
                        nfb, q.last_dt, gs.cell_dt.as<double>());
     HIP_TRY(hipGetLastError());
@@ -1275,7 +1089,7 @@ int brams_sur_step(const brams_chem_dev_args* a, const brams_sur_model* m, brams
     s.fallback_cell_attempts = fb_cell_att;
     s.fallback_cell_substeps = fb_cell_sub;
     s.fallback_failed_blocks = fb_failed;
-    s.fallback_wps = fb_form < 0 ? 0 : kListWps[fb_form];
+    s.fallback_wps = nfb > 0 ? brams::kCoopWavesPerSimd : 0;
     float ms;
     HIP_TRY(hipEventElapsedTime(&ms, ev[0], ev[1])); s.features_ms = ms;
     HIP_TRY(hipEventElapsedTime(&ms, ev[1], ev[2])); s.mlp_ms = ms;
@@ -1631,8 +1445,7 @@ void brams_chem_finalize(void) {
   DevBuf* bufs[] = {&g.sc_p, &g.sc_t, &g.sc_t_dyn, &g.met, &g.jphoto, &g.last_dt, &g.consts,
                     &g.sur_X, &g.sur_out, &g.sur_flag, &g.sur_list, &g.sur_chunk,
                     &g.sur_reason, &g.fb_dt, &g.fb_att, &g.mask_all, &g.sort_keys, &g.sort_ids,
-                    &g.sort_count, &g.sort_off, &g.order, &g.slab_lu, &g.slab_jac, &g.slab_rk,
-                    &g.slab_vec, &g.qcount, &g.tune_sc, &g.tune_dt};
+                    &g.sort_count, &g.sort_off, &g.order, &g.half_y};
   for (DevBuf* b : bufs) b->release();
   hipEvent_t* evs[] = {&g.ev0, &g.ev1, &g.evb, &g.evm, &g.sev[0], &g.sev[1], &g.sev[2], &g.sev[3],
                        &g.sev[4]};
@@ -1640,15 +1453,13 @@ void brams_chem_finalize(void) {
     if (*e) hipEventDestroy(*e);
     *e = nullptr;
   }
-  g.slab_slots = 0;
   g.init = false;
 }
 
 int brams_chem_set_form(int32_t form) {
   if (form < -1 || form >= kForms) return fail(-2, "kernel form %d out of range (-1..%d)", form, kForms - 1);
-  if (!kSlabEnabled && form >= 0 && form < kFormPerLane)
-    return fail(-6, "kernel form %d (slab) is switched off in this build", form);
-  if (form >= kFormPerLane && !form_built(form))
+  if (form >= 0 && form < kFirstForm) return fail(-6, "kernel form %d is switched off in this build", form);
+  if (form >= kFirstForm && !form_built(form))
     return fail(-6, "kernel form %d is not built into this %s library (lean build)", form, MECH_NAME);
   g.force_form = form;
   return 0;
@@ -1656,7 +1467,7 @@ int brams_chem_set_form(int32_t form) {
 
 int brams_chem_get_tuning(int32_t* form, float* ms, int32_t n) {
   if (!g.cur) return fail(-2, "no chemistry step has run");
-  if (form) *form = g.cur->form;
+  if (form) *form = kFirstForm;
   for (int f = 0; f < n && f < kForms && ms; ++f) ms[f] = g.cur->tune_ms[f];
   return kForms;
 }

@@ -1,48 +1,34 @@
-// Launch wrappers of the RODAS3 block kernels (rodas3_kernel.h): the
-// 128-lane forms (blocks of 65..127 cells), the 64-lane form at two waves
-// per SIMD, and the list forms of the surrogate's fallback.
+// Launch wrappers of the RODAS3 kernels of block 1 and of blocks of more than 64
+// cells.
 #include <hip/hip_runtime.h>
 
-#include "rodas3_kernel.h"
 #include "rodas3_launch.h"
+#ifdef BRAMS_MECH_COOP
+#include "rodas3_coop.h"
+#else
+#include "rodas3_lane.h"
+#endif
 
 namespace brams {
 
-hipError_t launch_rodas3_128(bool dyn, unsigned nblocks, const StepParams& p, int block0, hipStream_t st) {
-  if (nblocks == 0) return hipSuccess;
-  if (dyn)
-    hipLaunchKernelGGL((rodas3_blocks<128, true, false, 1>), dim3(nblocks), dim3(128), 0, st, p, block0);
-  else
-    hipLaunchKernelGGL((rodas3_blocks<128, false, false, 1>), dim3(nblocks), dim3(128), 0, st, p, block0);
+hipError_t launch_rodas3_first(const StepParams& p, hipStream_t st) {
+#ifdef BRAMS_MECH_COOP
+  hipLaunchKernelGGL((coop_blocks<kRodas3, true, true>), dim3(1), dim3(kCoopLanes), 0, st, p, 0);
+#else
+  // a block 1 of at most 64 cells leaves the second wave idle
+  hipLaunchKernelGGL((rodas3_blocks<128, true, 1>), dim3(1), dim3(128), 0, st, p, 0);
+#endif
   return hipGetLastError();
 }
 
-hipError_t launch_rodas3_64w2(unsigned nblocks, const StepParams& p, int block0, hipStream_t st) {
+hipError_t launch_rodas3_big(unsigned nblocks, const StepParams& p, int block0, hipStream_t st) {
   if (nblocks == 0) return hipSuccess;
-#ifdef BRAMS_MECH_LEAN
-  (void)p, (void)block0, (void)st;
-  return hipErrorInvalidValue;
+#ifdef BRAMS_MECH_COOP
+  hipLaunchKernelGGL((coop_blocks<kRodas3, false, true>), dim3(nblocks), dim3(kCoopLanes), 0, st, p, block0);
 #else
-  hipLaunchKernelGGL((rodas3_blocks<64, false, false, 2>), dim3(nblocks), dim3(64), 0, st, p, block0);
-  return hipGetLastError();
+  hipLaunchKernelGGL((rodas3_blocks<128, false, 1>), dim3(nblocks), dim3(128), 0, st, p, block0);
 #endif
-}
-
-hipError_t launch_rodas3_list(unsigned nblocks, const StepParams& p, hipStream_t st, int wps) {
-  if (nblocks == 0) return hipSuccess;
-  if (!p.cell_list) return hipErrorInvalidValue;
-#ifdef BRAMS_MECH_LEAN
-  (void)st, (void)wps;
-  return hipErrorInvalidValue;
-#else
-  if (wps == 2)
-    hipLaunchKernelGGL((rodas3_blocks<64, false, true, 2>), dim3(nblocks), dim3(64), 0, st, p, 0);
-  else if (wps == 1)
-    hipLaunchKernelGGL((rodas3_blocks<64, false, true, 1>), dim3(nblocks), dim3(64), 0, st, p, 0);
-  else
-    return hipErrorInvalidValue;
   return hipGetLastError();
-#endif
 }
 
 }  // namespace brams

@@ -46,6 +46,33 @@
 
 namespace brams {
 
+template <int WG>
+__device__ __forceinline__ void block_reduce(double& errmax, int& rej, int& fail,
+                                             double* s_err, int* s_rej, int* s_fail) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    errmax = fmax(errmax, __shfl_xor(errmax, off, 64));
+    rej |= __shfl_xor(rej, off, 64);
+    fail |= __shfl_xor(fail, off, 64);
+  }
+  if constexpr (WG > 64) {
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+      s_err[wave] = errmax;
+      s_rej[wave] = rej;
+      s_fail[wave] = fail;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WG / 64; ++w) {
+      errmax = fmax(errmax, s_err[w]);
+      rej |= s_rej[w];
+      fail |= s_fail[w];
+    }
+    __syncthreads();
+  }
+}
+
 // A lane's view of a 64-lane-interleaved array in LDS: element s at
 // p[s * 64], a ds access with the offset in its immediate field.
 struct Lanes {

@@ -311,21 +311,16 @@ int brams_chem_block_status(int32_t *attempts, int32_t *substeps, int32_t *faile
 int brams_chem_block_thresholds(int32_t *counts, int32_t max_nob);
 
 /*
- * Kernel form of the 64-cell blocks (no reference counterpart).  The forms
- * give bit-identical results and differ in speed: 3, 4 and 5 are the
- * per-lane kernel with the register budget of 1, 2 and 4 waves per SIMD;
- * 0..2 (the slab layouts: per-cell working set in registers, LDS and a
- * per-slot scratch slab, persistent workgroups over a device work queue) are
- * switched off in this build and refused (-6).  -1 (default): the first call
- * of each grid times every available form on a scratch copy of its state and
- * keeps the fastest for the grid.  The ROS2 step has forms 3 and 5 and tunes
- * its own choice the same way; with form 4 forced its calls fail (-6).  A
- * lean library (libbrams_chem_<mech>.so) has forms 3 and 5 only and refuses
- * form 4 here (-6).
+ * Kernel form of the 64-cell blocks (no reference counterpart): -1 (default)
+ * or one of 3, 4 and 5, kept for callers that force one.  All run the same
+ * kernel with the same results.  0..2 are refused (-6); the ROS2 step has no
+ * form 4 (its calls fail with -6 while it is forced), nor has a lean library
+ * (libbrams_chem_<mech>.so), which refuses it here (-6).
  */
 int brams_chem_set_form(int32_t form);
-/* The current grid's chosen form and the autotuner's timings (ms, one per
- * form, 0 if not timed) into ms[0..n); returns the number of forms. */
+/* The current grid's form, and the time (ms) of the 64-cell blocks in the
+ * grid's first call, for each form that the library has (0: none), into
+ * ms[0..n); returns the number of forms. */
 int brams_chem_get_tuning(int32_t *form, float *ms, int32_t n);
 
 /* Text of the last error (thread-local, never NULL). */
