@@ -21,7 +21,13 @@ FMA latencies when it is not.  Their rows of the matrix are assembled, and
 eliminated by the other pivots, on the other waves.
 """
 LDS_SLOTS = 320                  # 160 KB / (64 lanes x 8 bytes)
-CHUNK, KEEP = 12, 2              # operations between scheduling fences; chunks a value read is kept
+DENSE_PARTS = 3                  # phases of the dense wave's elimination
+# Operations between scheduling fences, chunks a value read is kept, and
+# chunks by which a read is issued ahead of its use.  Clocks move little with
+# them as long as the registers hold (RODAS3 on 164k cells, us a block's
+# attempt: 6/6/1 20.9, 6/6/2 20.8, 4/8/3 21.5, 8/4/2 21.6, 12/2/1 23.4); 24
+# and more operations spill (35 to 46).
+CHUNK, KEEP, AHEAD = 6, 6, 1
 
 
 def lit(x):
@@ -50,11 +56,11 @@ class Val:
 
 
 class Op:
-    __slots__ = ("wave", "phase", "outs", "ins", "text", "cost", "count_only")
+    __slots__ = ("wave", "phase", "outs", "ins", "text", "cost", "movable", "count_only")
 
-    def __init__(self, wave, phase, outs, ins, text, cost):
+    def __init__(self, wave, phase, outs, ins, text, cost, movable):
         self.wave, self.phase, self.outs, self.ins, self.text, self.cost = wave, phase, outs, ins, text, cost
-        self.count_only = False
+        self.movable, self.count_only = movable, False
 
 
 class Flow:
@@ -62,6 +68,7 @@ class Flow:
 
     def __init__(self):
         self.ops, self.n = [], 0
+        self.movable = False             # whether level() may move the operations added now
 
     def at(self, v, w):
         """First phase in which wave w can use v."""
@@ -77,12 +84,45 @@ class Flow:
         for _ in range(outs):
             res.append(Val(w, ph, "v%d" % self.n, home))
             self.n += 1
-        o = Op(w, ph, res, ins, text, cost)
+        o = Op(w, ph, res, ins, text, cost, self.movable)
         o.count_only = count_only
         for v in res:
             v.count_only = count_only
         self.ops.append(o)
         return res[0] if outs == 1 else res
+
+    def level(self, waves, least=16.0):
+        """Moves the movable operations out of the phases that they would
+        lengthen.  One may run in any phase from its inputs' to the last that
+        its consumers allow; it goes to the first where its wave has time left
+        beside the busiest wave, and else to where it adds the least."""
+        P = self.phases()
+        users = {}
+        for o in self.ops:
+            for v in o.ins:
+                if v.home not in ("free", "lds"):
+                    users.setdefault(id(v), []).append(o)
+        last = {}
+        load = [[0.0] * waves for _ in range(P)]
+        for o in reversed(self.ops):
+            if not o.movable:
+                if not o.count_only:
+                    load[o.phase][o.wave] += o.cost
+                last[id(o)] = o.phase
+                continue
+            last[id(o)] = min([P - 1] + [last[id(u)] - (0 if u.wave == o.wave else 1)
+                                         for v in o.outs for u in users.get(id(v), [])])
+        for o in self.ops:
+            if not o.movable:
+                continue
+            e, q = max([0] + [self.at(v, o.wave) for v in o.ins]), last[id(o)]
+
+            def extra(p):
+                return max(0.0, load[p][o.wave] + o.cost - max([least] + load[p]))
+            o.phase = min(range(e, q + 1), key=lambda p: (extra(p), p))
+            load[o.phase][o.wave] += o.cost
+            for v in o.outs:
+                v.phase = o.phase
 
     def settle(self):
         """Operations whose results wait in registers for a later phase move
@@ -185,13 +225,32 @@ class Builder:
         k = self.p.rk_reg[w].get(r)
         return free("rk[%d]" % k) if k is not None else self.rkl[r]
 
-    def state(self, name, s):
-        return free("%s[%d]" % (name, self.p.idx[s]))
+    def add_rate(self, w, acc, rows, r, t, last):
+        """Adds the rate t * last of reaction r to the sums of `rows`."""
+        m, f = self.m, self.f
+        fuse = len(rows) == 1 and abs(m.coef[(rows[0], r)]) == 1.0
+        if not fuse:
+            t = f.op(w, "{0} * {1}", [t, last])
+        for s in rows:
+            c = m.coef[(s, r)]
+            if fuse:
+                sg = "" if c > 0 else "-"
+                if s in acc:
+                    acc[s] = f.op(w, "fma(%s{0}, {1}, {2})" % sg, [t, last, acc[s]])
+                else:
+                    acc[s] = f.op(w, "%s({0} * {1})" % sg, [t, last])
+            elif s not in acc:
+                acc[s] = t if c == 1.0 else f.op(w, "%s * {0}" % lit(c), [t])
+            elif abs(c) == 1.0:
+                acc[s] = f.op(w, "{0} %s {1}" % ("+" if c > 0 else "-"), [acc[s], t])
+            else:
+                acc[s] = f.op(w, "fma(%s, {0}, {1})" % lit(c), [t, acc[s]])
 
     # f at the concentrations yv (species -> Val) for every wave's species
     def fun(self, yv):
         m, p, f = self.m, self.p, self.f
         out = {}
+        f.movable = True
         for w in range(p.waves):
             acc = {}
             for r in p.need[w]:
@@ -200,25 +259,10 @@ class Builder:
                 t = self.rk(w, r)
                 for s in rs[:-1]:
                     t = f.op(w, "{0} * {1}", [t, yv[s]])
-                fuse = len(rows) == 1 and abs(m.coef[(rows[0], r)]) == 1.0
-                if not fuse:
-                    t = f.op(w, "{0} * {1}", [t, yv[rs[-1]]])
-                for s in rows:
-                    c = m.coef[(s, r)]
-                    if fuse:
-                        sg = "" if c > 0 else "-"
-                        if s in acc:
-                            acc[s] = f.op(w, "fma(%s{0}, {1}, {2})" % sg, [t, yv[rs[-1]], acc[s]])
-                        else:
-                            acc[s] = f.op(w, "%s({0} * {1})" % sg, [t, yv[rs[-1]]])
-                    elif s not in acc:
-                        acc[s] = t if c == 1.0 else f.op(w, "%s * {0}" % lit(c), [t])
-                    elif abs(c) == 1.0:
-                        acc[s] = f.op(w, "{0} %s {1}" % ("+" if c > 0 else "-"), [acc[s], t])
-                    else:
-                        acc[s] = f.op(w, "fma(%s, {0}, {1})" % lit(c), [t, acc[s]])
+                self.add_rate(w, acc, rows, r, t, yv[rs[-1]])
             for s in p.own[w]:
                 out[s] = acc.get(s, free("0.0"))
+        f.movable = False
         return out
 
     # rows of the masked 1/(gamma h) I - J, {(I, J): Val} on the rows' waves
@@ -344,11 +388,15 @@ class Builder:
             for J, v in rows[I].items():
                 if J >= t0 and v.home == "reg" and v.wave != w:
                     v.store = self.cross
+        # The dense wave's elimination takes DENSE_PARTS phases, so that the
+        # first solve's forward levels can run beside it.
+        work = [sum(m.ns - 1 - K for K in range(t0, I)) + 12.0 + m.ns - I for I in range(t0, m.ns)]
         for I in range(t0, m.ns):
+            part = int(DENSE_PARTS * (sum(work[:I - t0]) + 0.5 * work[I - t0]) / sum(work))
             row0 = dict(rows[I])
             for J in sorted(rows[I]):
                 if J >= t0:
-                    rows[I][J] = self.move(w, rows[I][J], first=self.cross + 1)
+                    rows[I][J] = self.move(w, rows[I][J], first=self.cross + 1 + part)
             for K in range(t0, I):
                 if F[I][K]:
                     eliminate(I, K, w)
@@ -408,11 +456,13 @@ class Builder:
         return {self.m.pos[s]: x for s, x in v.items()}
 
     def attempt(self, solver):
-        f, st = self.f, self.state
+        f = self.f
+        # f(y0) shares the Jacobian's products, but beside all of a wave's
+        # matrix entries its sums do not fit the registers
         self.factor(self.matrix())
-        f0 = self.each(lambda w, s: st("f0", s))
-        # the first forward elimination waits until the U rows have crossed
-        k1 = self.spec(self.solve(self.rows(f0), first=2))
+        f0 = self.fun(self.yc)
+        # the first forward elimination runs beside the dense wave's
+        k1 = self.spec(self.solve(self.rows(f0), first=self.cross + 1))
         if solver == "ros2":
             yn = self.each(lambda w, s: f.op(w, "fma(kRos2GammaInv, {0}, {1})", [k1[s], self.yc[s]]))
             ft = self.fun(yn)
@@ -446,6 +496,7 @@ class Layout:
     """LDS slots of a section's exchanged values, and the section's code."""
 
     def __init__(self, flow, nfix, waves):
+        flow.level(waves)
         flow.settle()
         self.f, self.waves, self.P = flow, waves, flow.phases()
         vals = []
@@ -481,10 +532,12 @@ class Layout:
         self.slots = nfix + len(busy)
         self.writes = sum(1 for v, _ in vals)
 
-    def stats(self, cyc_op=4.0, sync=220.0):
-        """Modelled cycles: per phase the larger of the SIMDs' issue, the
-        waves' own issue and the LDS transfers, plus the barrier."""
+    def stats(self, sync=180.0):
+        """Modelled clocks of the section: per phase the longest of the waves
+        (latency of their operations and reads), the SIMDs (two waves' issue)
+        and the LDS transfers, plus the barrier."""
         ops = [[0.0] * self.waves for _ in range(self.P)]
+        reads = [[0] * self.waves for _ in range(self.P)]
         lds = [0] * self.P
         seen = set()
         for o in self.f.ops:
@@ -492,31 +545,28 @@ class Layout:
                 continue
             ops[o.phase][o.wave] += o.cost
             for v in o.ins:
-                if v.home == "free" or (v.wave == o.wave and not (v.home == "park" and o.phase > v.phase)):
-                    continue
-                k = (id(v), o.wave, o.phase)
-                if k not in seen:
-                    seen.add(k)
-                    lds[o.phase] += 1
+                if self.remote(v, o.wave, o.phase):
+                    k = (id(v), o.wave, o.phase)
+                    if k not in seen:
+                        seen.add(k)
+                        lds[o.phase] += 1
+                        reads[o.phase][o.wave] += 1
             for v in o.outs:
                 if v.slot is not None:
                     lds[o.phase] += 1
-        tot = 0.0
+                    reads[o.phase][o.wave] += 1
         rows = []
         for ph in range(self.P):
-            simd = max(sum(ops[ph][w] for w in range(s, self.waves, 4)) for s in range(4)) * cyc_op
-            wave = max(ops[ph]) * cyc_op * 1.3
-            l = lds[ph] * 4.0
-            t = max(simd, wave, l) + sync
-            rows.append((round(simd), round(wave), round(l)))
-            tot += t
-        return tot, rows, sum(lds)
+            wave = max(5.5 * a + 4.0 * r for a, r in zip(ops[ph], reads[ph]))
+            simd = max(sum(4.6 * ops[ph][w] + 3.0 * reads[ph][w] for w in range(s, self.waves, 4)) for s in range(4))
+            rows.append((round(wave), round(simd), round(2.8 * lds[ph])))
+        return sum(max(r) for r in rows) + sync * self.P, rows, sum(lds)
 
     def remote(self, v, w, ph):
         """Whether wave w reads v from LDS in phase ph."""
         return v.home != "free" and not (v.wave == w and not (v.home == "park" and ph > v.phase))
 
-    def emit(self, w, chunk=CHUNK, keep=KEEP):
+    def emit(self, w, chunk=CHUNK, keep=KEEP, ahead=AHEAD):
         """Code of wave w, phases separated by coop_barrier().
 
         A phase runs in chunks of `chunk` operations with a scheduling fence
@@ -549,15 +599,15 @@ class Layout:
 
             def issue(c):
                 for name, slot in reads[c]:
-                    out.append("  const double %s = S.at(%d);" % (name, slot))
-            if parts[0]:
-                issue(0)
+                    out.append("  const double %s = S.get(%d);" % (name, slot))
+            for c in range(min(ahead, len(parts))):
+                issue(c)
             for c, part in enumerate(parts):
-                if c + 1 < len(parts):
-                    issue(c + 1)
+                if c + ahead < len(parts):
+                    issue(c + ahead)
                 for o in part:
                     if o.count_only:
-                        args = [v.expr if not self.remote(v, w, ph) else names[c].get(id(v), "S.at(%d)" % v.slot)
+                        args = [v.expr if not self.remote(v, w, ph) else names[c].get(id(v), "S.get(%d)" % v.slot)
                                 for v in o.ins]
                         out.append("  " + o.text.format(*args))
                         continue
@@ -582,7 +632,7 @@ class Layout:
                     for v in o.outs:
                         if v.slot is not None and v.store is None:
                             only_count = all(v_users_count(self.f, v))
-                            st = "S.at(%d) = %s;" % (v.slot, v.expr)
+                            st = "S.put(%d, %s);" % (v.slot, v.expr)
                             out.append("  if constexpr (COUNT) { %s }" % st if only_count else "  " + st)
                 if c + 1 < len(parts):
                     out.append("  coop_fence();")
@@ -591,7 +641,7 @@ class Layout:
                     for v in o.outs:
                         if v.store == ph:
                             only_count = all(v_users_count(self.f, v))
-                            st = "S.at(%d) = %s;" % (v.slot, v.expr)
+                            st = "S.put(%d, %s);" % (v.slot, v.expr)
                             out.append("  if constexpr (COUNT) { %s }" % st if only_count else "  " + st)
             if ph + 1 < self.P:
                 out.append("  coop_barrier();")
@@ -648,10 +698,6 @@ def emit(m, plan, reactions, rate_line, name, mech_name):
         lay = Layout(b.f, plan.nfix, W)
         secs[solver] = lay
         slots = max(slots, lay.slots)
-    fb = Builder(plan)
-    f0 = fb.fun(fb.yc)
-    flay = Layout(fb.f, plan.nfix, W)
-    assert flay.P == 1
     # rate constants on their way from the wave that evaluates them to the
     # registers of those that use them: the exchange slots, free at that time
     reg_rk = sorted({r for d in plan.rk_reg for r in d})
@@ -699,27 +745,17 @@ def emit(m, plan, reactions, rate_line, name, mech_name):
         w_("    (void)M; (void)H2O; (void)lnT; (void)J;")
         for r in shares[w]:
             sl = plan.rkslot.get(r, tmp.get(r))
-            w_("    S.at(%d) = %s;" % (sl, rate_line(r)))
+            w_("    S.put(%d, %s);" % (sl, rate_line(r)))
         w_("  }")
         w_("  static __device__ __forceinline__ void load_rk(const CoopLds& S, double* rk) {")
         if not plan.rk_reg[w]:
             w_("    rk[0] = 0.0;")
         for r, k in sorted(plan.rk_reg[w].items(), key=lambda t: t[1]):
-            w_("    rk[%d] = S.at(%d);" % (k, tmp[r]))
-        w_("  }")
-        w_("  // f (rates.f90, fexchem.f90) of this wave's species at the published concentrations")
-        w_("  static __device__ __forceinline__ void fun0(const CoopLds& S, const double* rk, double* f0) {")
-        L.extend("  " + x for x in flay.emit(w))
-        for k, s in enumerate(own):
-            v = f0[s]
-            e = v.expr
-            if v.home == "lds":
-                e = "S.at(%d)" % v.slot
-            w_("    f0[%d] = %s;" % (k, e))
+            w_("    rk[%d] = S.get(%d);" % (k, tmp[r]))
         w_("  }")
         for solver in ("rodas3", "ros2"):
             w_("  template <bool DYN, bool COUNT>")
-            w_("  static __device__ __forceinline__ void %s(const CoopLds& S, const double* f0, const double* rk," % solver)
+            w_("  static __device__ __forceinline__ void %s(const CoopLds& S, const double* rk," % solver)
             w_("      double igdt, double dti, unsigned* mw, bool dyn, const double* atol, const double* rtol,")
             w_("      double* yn, double& e, unsigned* viol) {")
             L.extend("  " + x for x in secs[solver].emit(w))

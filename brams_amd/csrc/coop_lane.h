@@ -27,7 +27,14 @@ struct CoopLds {
       asm volatile("" : "+v"(base[k]));
     }
   }
-  __device__ __forceinline__ CoopLdsDouble& at(int slot) const { return base[slot >> 7][(slot & 127) * 64]; }
+  // Volatile: a value that is read twice is meant to be read twice.  The
+  // compiler would keep the first copy in a register (and spill it), and
+  // would merge two reads into a ds_read2st64_b64, which moves 123 bytes a
+  // clock where ds_read_b64 moves 184 (eight waves reading).
+  __device__ __forceinline__ double get(int slot) const {
+    return *(const volatile CoopLdsDouble*)&base[slot >> 7][(slot & 127) * 64];
+  }
+  __device__ __forceinline__ void put(int slot, double v) const { base[slot >> 7][(slot & 127) * 64] = v; }
 };
 
 // no instruction moves across this when the compiler schedules

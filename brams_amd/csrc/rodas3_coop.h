@@ -16,9 +16,12 @@
 // as its busiest wave; one workgroup fills a CU (153 KB of LDS, 256 registers
 // a lane at two waves per SIMD), so nothing overlaps another block's.
 // Measured on 1.6M cells of RELACS_TUV, one step at the reference's
-// tolerances (16.2 attempts a cell): 34.8 ms, 22 us a block's attempt.  The
-// kernel it replaces kept one lane's whole state in registers and scratch: it
-// read and wrote 63 KB of spilled state a cell-attempt and took 353 ms.
+// tolerances (16.2 attempts a cell): 30.4 ms, 19 us a block's attempt, of
+// which a wave is busy for half (a wave's registers hold its rows of the
+// matrix with little to spare, so the reads of LDS run only a few operations
+// ahead).  The kernel it replaces kept one lane's whole state in registers and
+// scratch: it read and wrote 63 KB of spilled state a cell-attempt and took
+// 353 ms.
 //
 // Blocks of 65..127 cells (the first ones of a grid whose cell count is no
 // multiple of 64) run as two halves in turn inside each attempt, with their
@@ -152,7 +155,7 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
   int* mbits = reinterpret_cast<int*>(lds + MECH_COOP_MSLOT * 64);
   (void)vbits;
 
-  double y[WV::kOwn + 1], f0[WV::kOwn + 1], yn[WV::kOwn + 1], rk[WV::kRk];
+  double y[WV::kOwn + 1], yn[WV::kOwn + 1], rk[WV::kRk];
   double* half = nullptr;                                 // [half][buffer][species][64]
   int cur = 0;
   if (COUNT && halves > 1) half = p.half_y + (long long)slot * (4 * MECH_NS * 64) + lane;
@@ -178,7 +181,7 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
   // the block's concentrations live in LDS, where every wave reads them
   auto publish = [&](const double* v) {
 #pragma unroll
-    for (int k = 0; k < WV::kOwn; ++k) S.at(WV::own[k]) = v[k];
+    for (int k = 0; k < WV::kOwn; ++k) S.put(WV::own[k], v[k]);
   };
   // rate coefficients of the cells in q, spread over the waves
   auto kinetic = [&]() {
@@ -214,7 +217,6 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
     kinetic();
   }
 
-  bool fresh = true;                                      // f(y0) is still to be evaluated
   while (coop_uniform(time_c + 1.0e-8 < time_f ? 1 : 0)) {
     ++natt;
     // 1/(gamma h): RODAS3 gamma = 1/2 (rodas3:462), ROS2 ros_dyndt:387
@@ -231,10 +233,7 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
 #pragma unroll
         for (int k = 0; k < WV::kOwn; ++k) y[k] = half[((2 * h + cur) * MECH_NS + WV::own[k]) * 64];
         kinetic();
-        fresh = true;
       }
-      if (fresh) WV::fun0(S, rk, f0);
-      fresh = false;
       double e = 0.0;
       unsigned viol[MECH_COOP_VWORDS] = {};
       if (COUNT) {
@@ -242,9 +241,9 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
           for (int k = 0; k < MECH_COOP_VWORDS; ++k) vbits[k * 64] = 0;
       }
       if constexpr (SOLVER == kRos2)
-        WV::template ros2<DYN, COUNT>(S, f0, rk, igdt, dti, mw, false, p.atol, p.rtol, yn, e, viol);
+        WV::template ros2<DYN, COUNT>(S, rk, igdt, dti, mw, false, p.atol, p.rtol, yn, e, viol);
       else
-        WV::template rodas3<DYN, COUNT>(S, f0, rk, igdt, dti, mw, DYN && h == 0, p.atol, p.rtol, yn, e, viol);
+        WV::template rodas3<DYN, COUNT>(S, rk, igdt, dti, mw, DYN && h == 0, p.atol, p.rtol, yn, e, viol);
       if (COUNT) {
         for (int k = 0; k < MECH_COOP_VWORDS; ++k) atomicOr(&vbits[k * 64], (int)viol[k]);
         if (halves > 1) {
@@ -253,11 +252,11 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
         }
       }
       // error over the species: every wave adds the waves' parts in the same order
-      S.at(MECH_COOP_ESLOT + wave) = e;
+      S.put(MECH_COOP_ESLOT + wave, e);
       coop_barrier();
-      e = S.at(MECH_COOP_ESLOT);
+      e = S.get(MECH_COOP_ESLOT);
 #pragma unroll
-      for (int w = 1; w < MECH_COOP_WAVES; ++w) e = e + S.at(MECH_COOP_ESLOT + w);
+      for (int w = 1; w < MECH_COOP_WAVES; ++w) e = e + S.get(MECH_COOP_ESLOT + w);
       // a zero pivot makes its species' error non-finite (its reciprocal
       // enters every solve), so this also ends a block there, where the
       // reference aborts the process
@@ -276,27 +275,26 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
     double err;
     const double dt_new = coop_controller<SOLVER>(errmax, dt, dt_min, dt_max, err);
     const bool rej = err - 1.0e-8 > 1.0;
+    // One path for accepted and rejected attempts: a taken branch costs a
+    // miss of the instruction cache, which the attempt's code has swept.  So a
+    // rejected attempt evaluates the Jacobian and f(y0) again, to the same
+    // values.
     const int act = coop_uniform(fail ? 2 : (rej && dt_new > dt_min) ? 1 : 0);
-    if (act == 2) {
+    if (__builtin_expect(act == 2, 0)) {
       failed = 1;
       break;
     }
-    if (act == 1) {
-      dt = dt_new;
-      continue;
+    if (act == 0) {
+      // an error above 1 accepted anyway: dt reached dt_min (rodas3:671-676)
+      forced = rej ? fmaxf(forced, (float)err) : forced;
+      time_c = time_c + dt;
+      last_dt = time_c < time_f ? dt_new : last_dt;
+      ++nsub;
+      cur ^= 1;
+      if (halves == 1) publish(yn);
     }
-    // an error above 1 accepted anyway: dt reached dt_min (rodas3:671-676)
-    if (rej) forced = fmaxf(forced, (float)err);
-    time_c = time_c + dt;
-    dt = fmin(dt_new, time_f - time_c);
-    if (time_c < time_f) last_dt = dt_new;
-    ++nsub;
-    cur ^= 1;
-    if (halves == 1) {
-      publish(yn);
-      coop_barrier();
-      fresh = true;
-    }
+    dt = act == 0 ? fmin(dt_new, time_f - time_c) : dt_new;
+    coop_barrier();
   }
 
   // ---- write-back, rodas3:713-798
@@ -307,7 +305,7 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
       for (int k = 0; k < WV::kOwn; ++k) y[k] = half[((2 * h + cur) * MECH_NS + WV::own[k]) * 64];
     } else {
 #pragma unroll
-      for (int k = 0; k < WV::kOwn; ++k) y[k] = S.at(WV::own[k]);
+      for (int k = 0; k < WV::kOwn; ++k) y[k] = S.get(WV::own[k]);
     }
     if (!q.act) continue;
     const double volmol_i = 1.0 / q.volmol;

@@ -67,7 +67,8 @@ namespace brams {
 struct CoopLds {
   double* column;
   explicit CoopLds(double* c) : column(c) {}
-  double& at(int slot) const { return column[slot * 64]; }
+  double get(int slot) const { return column[slot * 64]; }
+  void put(int slot, double v) const { column[slot * 64] = v; }
 };
 static void coop_fence() {}
 static void coop_opaque(unsigned&) {}

@@ -55,8 +55,8 @@ def run(coop_host, wl, atol, rtol, ros2):
     return sc, dt, counts, mw, f
 
 
-# (columns, levels): blocks of 1, 6, 65 and 70 cells, and two blocks of 66
-@pytest.mark.parametrize("nx,ny,nz", [(1, 1, 1), (3, 2, 1), (13, 5, 1), (7, 5, 2), (11, 6, 2)])
+# blocks of 1, 6 and 65 cells, and two blocks of 66
+@pytest.mark.parametrize("nx,ny,nz", [(1, 1, 1), (3, 2, 1), (13, 5, 1), (11, 6, 2)])
 @pytest.mark.parametrize("solver", ["rodas3", "ros2"])
 def test_blocks_match_oracle(coop_host, nx, ny, nz, solver):
     wl = make_workload(Grid(nx, ny, nz, dtlt=30.0), seed=nx, sza="random")
