@@ -1381,11 +1381,13 @@ int brams_chem_tuv_jphoto_device(const brams_tuv_map_args* a) {
   const long long ni = a->iz - a->ia + 1, nj = a->jz - a->ja + 1;
   const long long npts = (long long)a->m1 * ni * nj, n3d = (long long)a->m1 * a->m2 * a->m3;
   HIP_TRY(hipEventRecord(g.ev0, st));
-  const unsigned tiles = (unsigned)((npts + 255) / 256), chunk = (tiles + brams::kXcds - 1) / brams::kXcds;
-  hipLaunchKernelGGL(brams::tuv_map_interior, dim3(chunk * brams::kXcds), dim3(256), 0, st, p, npts, chunk);
-  HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(brams::jphoto_relations_outside, dim3((unsigned)((n3d + 255) / 256)), dim3(256), 0, st, p,
-                     n3d);
+  brams::TuvTiles q{};
+  q.lev = (unsigned)((a->m1 + brams::kTuvLevels - 1) / brams::kTuvLevels);
+  q.col = (unsigned)((ni + brams::kTuvCols - 1) / brams::kTuvCols);
+  q.tiles = (unsigned)(q.lev * q.col * nj);
+  q.chunk = (q.tiles + brams::kXcds - 1) / brams::kXcds;
+  const unsigned frame = (unsigned)((n3d - npts + 255) / 256);
+  hipLaunchKernelGGL(brams::tuv_map, dim3(q.chunk * brams::kXcds + frame), dim3(256), 0, st, p, q);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(g.ev1, st));
   HIP_TRY(hipStreamSynchronize(st));

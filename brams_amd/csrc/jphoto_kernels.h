@@ -13,9 +13,7 @@
 //
 // The host resolves xRef into src[n]: the last k that writes jphoto index n
 // (later reactions overwrite earlier ones), -1 where none does (that entry
-// keeps its value).  One thread per point (level fastest, so a wave writes
-// consecutive 136-byte rows of jphoto); its reads of valJLoc at one level are
-// strided, and the neighbouring columns' waves use the rest of each line.
+// keeps its value).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -33,52 +31,89 @@ struct TuvMapParams {
 
 // Workgroups are dealt to the eight XCDs in turn (workgroup w on XCD w % 8),
 // each with its own L2.  Workgroup w takes tile (w % 8) * chunk + w / 8, so
-// every XCD works through one contiguous run of columns, and the 16
-// neighbouring columns that share a 128-byte line of valJLoc are read through
-// one L2 instead of up to eight.
+// every XCD works through one contiguous run of tiles, and neighbouring tiles,
+// which share 128-byte lines of both arrays, go through one L2.
 constexpr int kXcds = 8;
-__device__ __forceinline__ long long xcd_tile(unsigned chunk) {
-  return (long long)(blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds;
+__device__ __forceinline__ unsigned xcd_tile(unsigned chunk) {
+  return (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds;
 }
 
-// interior columns: the mapping, then the relations; launched with
-// kXcds * chunk workgroups of 256 (chunk = ceil(tiles / kXcds))
-__global__ __launch_bounds__(256) void tuv_map_interior(TuvMapParams p, long long npts, unsigned chunk) {
-  const long long t = xcd_tile(chunk) * 256 + threadIdx.x;
-  if (t >= npts) return;
-  const int ni = p.iz - p.ia + 1, nj = p.jz - p.ja + 1;
-  const int L = (int)(t % p.m1);
-  const long long col = t / p.m1;
-  const int ii = (int)(col % ni), jj = (int)(col / ni);
-  const long long o = L + (long long)p.m1 * ((p.ia - 1 + ii) + (long long)p.m2 * (p.ja - 1 + jj));
-  const int mz = L == 0 ? 0 : L - 1;                 // level 1 repeats level 2
-  double v[MECH_NPHOT];
-#pragma unroll
-  for (int n = 0; n < MECH_NPHOT; ++n) {
-    const int k = p.src[n];
-    v[n] = k >= 0 ? p.valj[ii + (long long)ni * (jj + (long long)nj * (k + (long long)p.kj * mz))]
-                  : p.jphoto[n + (long long)MECH_NPHOT * o];
-  }
-  mech_j_relations(v);
-#pragma unroll
-  for (int n = 0; n < MECH_NPHOT; ++n) p.jphoto[n + (long long)MECH_NPHOT * o] = v[n];
-}
+// valJLoc has the column fastest, jphoto the rate and then the level, so the
+// mapping is a transpose.  A tile is kTuvCols neighbouring columns times
+// kTuvLevels levels, one thread a point: a wave reads two runs of 256 bytes of
+// valJLoc, the relations apply in registers, and the rates go through LDS to
+// be written in runs of kTuvLevels * MECH_NPHOT values (1088 bytes).  The odd
+// row length keeps the LDS columns on different banks.  HBM bound: 200x200x40
+// (453 MB) takes 107 us of kernel, 4.2 TB/s where a large copy reaches 4.65;
+// with a thread writing its 136 bytes directly, which touched 64 lines with
+// every load and store, 152 us.
+constexpr int kTuvCols = 32, kTuvLevels = 8, kTuvRow = kTuvLevels * MECH_NPHOT + (MECH_NPHOT * kTuvLevels % 2 == 0);
 
-// points outside the interior columns: the relations alone (the entries they
-// do not set are written back unchanged)
-__global__ __launch_bounds__(256) void jphoto_relations_outside(TuvMapParams p, long long n3d) {
-  const long long o = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (o >= n3d) return;
-  const long long col = o / p.m1;
-  const int i = (int)(col % p.m2) + 1, j = (int)(col / p.m2) + 1;
-  if (i >= p.ia && i <= p.iz && j >= p.ja && j <= p.jz) return;
-  double* jp = p.jphoto + (long long)MECH_NPHOT * o;
+struct TuvTiles {
+  unsigned lev, col, tiles, chunk;     // tiles along the levels and the columns of one j, in all, per XCD
+};
+
+__device__ __forceinline__ void tuv_relations_at(double* jp) {
   double v[MECH_NPHOT];
 #pragma unroll
   for (int n = 0; n < MECH_NPHOT; ++n) v[n] = jp[n];
   mech_j_relations(v);
 #pragma unroll
   for (int n = 0; n < MECH_NPHOT; ++n) jp[n] = v[n];
+}
+
+// Interior columns: the mapping, then the relations (kXcds * chunk
+// workgroups).  The workgroups after them take the other columns, a thread a
+// point: the relations alone, the entries they do not set unchanged.
+__global__ __launch_bounds__(256) void tuv_map(TuvMapParams p, TuvTiles q) {
+  __shared__ double s[kTuvCols * kTuvRow];
+  const int ni = p.iz - p.ia + 1, nj = p.jz - p.ja + 1;
+  if (blockIdx.x >= kXcds * q.chunk) {
+    const long long t = (long long)(blockIdx.x - kXcds * q.chunk) * 256 + threadIdx.x;
+    long long c = t / p.m1;                          // column of the frame, j rows from the bottom
+    const long long below = (long long)(p.ja - 1) * p.m2, side = p.m2 - ni;
+    if (c >= (long long)p.m2 * p.m3 - (long long)ni * nj) return;
+    if (c >= below) {
+      const long long r = c - below;                 // beside the interior's rows, then above them
+      if (r < side * nj) {
+        const long long i = r % side;
+        c = (p.ja - 1 + r / side) * p.m2 + (i < p.ia - 1 ? i : i + ni);
+      } else {
+        c = (long long)p.jz * p.m2 + (r - side * nj);
+      }
+    }
+    tuv_relations_at(p.jphoto + (long long)MECH_NPHOT * (t % p.m1 + p.m1 * c));
+    return;
+  }
+  const unsigned tile = xcd_tile(q.chunk);
+  if (tile >= q.tiles) return;
+  const int L0 = (int)(tile % q.lev) * kTuvLevels;
+  const unsigned tc = tile / q.lev;
+  const int i0 = (int)(tc % q.col) * kTuvCols, jj = (int)(tc / q.col);
+  const int nl = min(kTuvLevels, p.m1 - L0), nc = min(kTuvCols, ni - i0);
+  const int c = threadIdx.x % kTuvCols, l = threadIdx.x / kTuvCols;
+  // first value of the tile's column 0
+  double* out = p.jphoto + (long long)MECH_NPHOT * (L0 + (long long)p.m1 * ((p.ia - 1 + i0) + (long long)p.m2 * (p.ja - 1 + jj)));
+  const long long column = (long long)MECH_NPHOT * p.m1;
+  if (c < nc && l < nl) {
+    const int mz = L0 + l == 0 ? 0 : L0 + l - 1;     // level 1 repeats level 2
+    double v[MECH_NPHOT];
+#pragma unroll
+    for (int n = 0; n < MECH_NPHOT; ++n) {
+      const int k = p.src[n];
+      v[n] = k >= 0 ? p.valj[i0 + c + (long long)ni * (jj + (long long)nj * (k + (long long)p.kj * mz))]
+                    : out[c * column + l * MECH_NPHOT + n];
+    }
+    mech_j_relations(v);
+#pragma unroll
+    for (int n = 0; n < MECH_NPHOT; ++n) s[c * kTuvRow + l * MECH_NPHOT + n] = v[n];
+  }
+  __syncthreads();
+  const unsigned run = (unsigned)nl * MECH_NPHOT, all = run * (unsigned)nc;
+  for (unsigned e = threadIdx.x; e < all; e += 256) {
+    const unsigned ec = e / run, er = e - ec * run;
+    out[ec * column + er] = s[ec * kTuvRow + er];
+  }
 }
 
 }  // namespace brams

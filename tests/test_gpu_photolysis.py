@@ -54,6 +54,27 @@ def test_tuv_mapping_16x16x10_bit_identical(kind):
     assert np.array_equal(gpu, ref)
 
 
+@pytest.mark.parametrize("nx,ny,nz,lo,hi", [(1, 1, 1, 0, 0), (33, 3, 7, 0, 0), (31, 2, 6, 2, 1), (64, 5, 14, 1, 3)])
+def test_tuv_mapping_ragged_tiles_bit_identical(nx, ny, nz, lo, hi):
+    """Columns and levels that leave part of a tile empty, interiors that
+    start and end off the grid's second column, and rates that no reaction
+    writes (they keep their values)."""
+    print("case tuv mapping %dx%dx%d +%d +%d" % (nx, ny, nz, lo, hi), flush=True)
+    grid = Grid(nx, ny, nz)
+    grid.ia, grid.iz = grid.ia + lo, grid.iz + lo
+    grid.ja, grid.jz = grid.ja + hi, grid.jz + hi
+    grid.m2, grid.m3 = grid.m2 + lo + hi, grid.m3 + lo + hi
+    kj, kz = 20, grid.m1 + 2
+    rng = np.random.default_rng(nx)
+    valj = np.asfortranarray(rng.uniform(0.0, 1e-2, (nx, ny, kj, kz)))
+    before = np.asfortranarray(rng.uniform(1e-6, 1e-3, (NP, grid.m1, grid.m2, grid.m3)))
+    xref = np.zeros(kj, np.int32)
+    xref[[1, 4, 5, 9, 12, 17, 19]] = [13, 9, 15, 1, 17, 13, 2]
+    rc, gpu, _ = _run(grid, valj, xref, before)
+    assert rc == 0
+    assert np.array_equal(gpu, O.tuv_jphoto(grid, valj, xref, before))
+
+
 def test_tuv_mapping_200x200x40_bit_identical():
     print("case tuv mapping 200x200x40 kj 80 kz 125", flush=True)
     grid = Grid(200, 200, 40)
