@@ -102,7 +102,20 @@ __global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
   f32x16_t acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  for (int k = kbeg; k < kend; k += 16) {
+  // four steps' operands in flight: the loop is bound by the latency of its
+  // loads (8192x256x256: 13.6 us a product with one step's)
+  int k = kbeg;
+  for (; k + 64 <= kend; k += 64) {
+    bf16x8_t a[4], b[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      a[q] = load_frag<LA>(g.A, g.lda, arow, k + 16 * q + koff);
+      b[q] = load_frag<LB>(g.B, g.ldb, bcol, k + 16 * q + koff);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[q], b[q], acc, 0, 0, 0);
+  }
+  for (; k < kend; k += 16) {
     const bf16x8_t a = load_frag<LA>(g.A, g.lda, arow, k + koff);
     const bf16x8_t b = load_frag<LB>(g.B, g.ldb, bcol, k + koff);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
@@ -136,17 +149,28 @@ __global__ void fill_f32(float* p, long long n, float v) {
   for (; i < n; i += (long long)gridDim.x * blockDim.x) p[i] = v;
 }
 
-// column sums out[n] += sum_m X[m][n] over a 64-column x 512-row tile per
-// block (out must be zeroed first); 4 row phases of 64 lanes each
+// column sums out[n] += sum_m X[m][n] over a 64-column x kColsumRows-row tile
+// per block (out must be zeroed first); 4 row phases of 64 lanes each.  Bound
+// by the latency of a thread's chain of loads: 64 rows a block, 16 loads a
+// thread in flight together; with 512 rows 8192x256 took 32 us.
+constexpr int kColsumRows = 64;
 __global__ __launch_bounds__(256) void colsum_f32(const float* X, long long ld, int M, int N,
                                                   float* out) {
   __shared__ float part[4][64];
   const int c = threadIdx.x & 63, ph = threadIdx.x >> 6;
   const int n = blockIdx.x * 64 + c;
-  const int m0 = blockIdx.y * 512;
+  const int m0 = blockIdx.y * kColsumRows;
   float s = 0.f;
-  if (n < N)
-    for (int m = m0 + ph; m < min(M, m0 + 512); m += 4) s += X[(long long)m * ld + n];
+  if (n < N) {
+    float v[kColsumRows / 4];
+#pragma unroll
+    for (int q = 0; q < kColsumRows / 4; ++q) {
+      const int m = m0 + ph + 4 * q;
+      v[q] = m < M ? X[(long long)m * ld + n] : 0.f;
+    }
+#pragma unroll
+    for (int q = 0; q < kColsumRows / 4; ++q) s += v[q];
+  }
   part[ph][c] = s;
   __syncthreads();
   if (ph == 0 && n < N) atomicAdd(&out[n], part[0][c] + part[1][c] + part[2][c] + part[3][c]);
@@ -161,19 +185,22 @@ __device__ __forceinline__ float block_sum_256(float v, float* sh) {
 }
 
 // MSE on the first nvalid outputs: d = 2 (o - y) / (M nvalid); padded
-// columns get 0.  The loss sum is reduced per block, one atomic per block.
+// columns get 0.  The loss sum is reduced per block, one atomic per block: all
+// go to one address, so the blocks are few (kMseBlocks at most; a block to
+// every 256 values of 8192x64 took 29 us).
+constexpr int kMseBlocks = 128;
 __global__ __launch_bounds__(256) void mse_grad(const float* out, const float* y, int M, int npad,
                                                 int nvalid, float* d, __bf16* dbf, float* loss) {
   __shared__ float sh[4];
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   float e2 = 0.f;
-  if (i < (long long)M * npad) {
+  const long long all = (long long)M * npad, step = (long long)gridDim.x * blockDim.x;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < all; i += step) {
     const int n = (int)(i % npad);
     float v = 0.f;
     if (n < nvalid) {
       const float e = out[i] - y[i];
       v = 2.0f * e / ((float)M * (float)nvalid);
-      e2 = e * e / ((float)M * (float)nvalid);
+      e2 += e * e / ((float)M * (float)nvalid);
     }
     d[i] = v;
     dbf[i] = to_bf16(v);

@@ -157,7 +157,7 @@ int choose_ksplit(int B) {
 int backward(brams_mlp* m, const __bf16* X, const float* Y, int B, hipStream_t st) {
   SUR_TRY(fill(m->g, m->np, 0.f, st));
   const long long nout = (long long)B * BRAMS_SUR_NOUT_PAD;
-  hipLaunchKernelGGL(brams::mse_grad, dim3((unsigned)((nout + 255) / 256)), dim3(256), 0, st, m->out,
+  hipLaunchKernelGGL(brams::mse_grad, dim3((unsigned)std::min<long long>((nout + 255) / 256, brams::kMseBlocks)), dim3(256), 0, st, m->out,
                      Y, B, BRAMS_SUR_NOUT_PAD, BRAMS_SUR_NOUT, m->dout_f, m->dout_b, m->loss);
   SUR_TRY(hipGetLastError());
   const int ks = choose_ksplit(B);
@@ -179,7 +179,7 @@ int backward(brams_mlp* m, const __bf16* X, const float* Y, int B, hipStream_t s
     }
     // db[o] = sum_b d[b][o]
     {
-      dim3 grid((m->dout[l] + 63) / 64, (B + 511) / 512);
+      dim3 grid((m->dout[l] + 63) / 64, (B + brams::kColsumRows - 1) / brams::kColsumRows);
       hipLaunchKernelGGL(brams::colsum_f32, grid, dim3(256), 0, st, dcur_f, ldd, B, m->dout[l],
                          m->g + m->boff[l]);
       SUR_TRY(hipGetLastError());
