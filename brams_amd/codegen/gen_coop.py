@@ -25,8 +25,8 @@ DENSE_PARTS = 3                  # phases of the dense wave's elimination
 # Operations between scheduling fences, chunks a value read is kept, and
 # chunks by which a read is issued ahead of its use.  Clocks move little with
 # them as long as the registers hold (RODAS3 on 164k cells, us a block's
-# attempt: 6/6/1 20.9, 6/6/2 20.8, 4/8/3 21.5, 8/4/2 21.6, 12/2/1 23.4); 24
-# and more operations spill (35 to 46).
+# attempt: 6/6/1 21.0, 6/6/2 20.8, 6/6/3 21.3, 4/8/2 21.3, 8/4/2 21.6, 3/8/4
+# 22.2); chunks of 24 and more spill.
 CHUNK, KEEP, AHEAD = 6, 6, 1
 
 

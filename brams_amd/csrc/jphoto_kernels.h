@@ -44,9 +44,9 @@ __device__ __forceinline__ unsigned xcd_tile(unsigned chunk) {
 // valJLoc, the relations apply in registers, and the rates go through LDS to
 // be written in runs of kTuvLevels * MECH_NPHOT values (1088 bytes).  The odd
 // row length keeps the LDS columns on different banks.  HBM bound: 200x200x40
-// (453 MB) takes 107 us of kernel, 4.2 TB/s where a large copy reaches 4.65;
-// with a thread writing its 136 bytes directly, which touched 64 lines with
-// every load and store, 152 us.
+// (453 MB) takes 117 us with its launch, 3.9 TB/s where a large copy reaches
+// 4.65; with a thread writing its 136 bytes directly, which touched 64 lines
+// with every load and store, 162 us.
 constexpr int kTuvCols = 32, kTuvLevels = 8, kTuvRow = kTuvLevels * MECH_NPHOT + (MECH_NPHOT * kTuvLevels % 2 == 0);
 
 struct TuvTiles {

@@ -16,7 +16,7 @@
 // as its busiest wave; one workgroup fills a CU (153 KB of LDS, 256 registers
 // a lane at two waves per SIMD), so nothing overlaps another block's.
 // Measured on 1.6M cells of RELACS_TUV, one step at the reference's
-// tolerances (16.2 attempts a cell): 30.4 ms, 19 us a block's attempt, of
+// tolerances (16.2 attempts a cell): 30.9 ms, 20.6 us a block's attempt, of
 // which a wave is busy for half (a wave's registers hold its rows of the
 // matrix with little to spare, so the reads of LDS run only a few operations
 // ahead).  The kernel it replaces kept one lane's whole state in registers and
