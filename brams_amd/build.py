@@ -1,7 +1,8 @@
 """Build every native piece in-tree.
 
   1. brams_amd/codegen/gen_mech.py  -> brams_amd/csrc/generated/<mech>_gen.h
-                                       (+ _slab.h, _flops.json) per mechanism
+                                       (+ _slab.h, _coop.h, _qssa.h,
+                                       _flops.json) per mechanism
   2. hipcc (gfx950)                 -> brams_amd/libbrams_chem.so (RELACS_TUV)
                                        and libbrams_chem_<mech>.so for the
                                        other mechanisms (lean kernel set)
@@ -66,10 +67,14 @@ def mech_flags(mech):
         return []
     coop = ['-DBRAMS_MECH_COOP="generated/%s_coop.h"' % mech] if mech in COOP_MECHS else []
     return ['-DBRAMS_MECH_GEN="generated/%s_gen.h"' % mech,
-            '-DBRAMS_MECH_SLAB="generated/%s_slab.h"' % mech, "-DBRAMS_MECH_LEAN"] + coop
+            '-DBRAMS_MECH_SLAB="generated/%s_slab.h"' % mech,
+            '-DBRAMS_MECH_QSSA="generated/%s_qssa.h"' % mech, "-DBRAMS_MECH_LEAN"] + coop
 
 
 def unit_deps(unit, mech):
+    if unit == "qssa_launch.hip":
+        return ["rodas3_kernel.h", "rodas3_launch.h", "coop_lane.h", "mech_families.h", "mechanism.h",
+                "generated/%s_gen.h" % mech, "generated/%s_qssa.h" % mech]
     if unit in _KERNEL_UNITS:
         coop = ["generated/%s_coop.h" % mech] if mech in COOP_MECHS else []
         return _KERNEL_DEPS + ["generated/%s_gen.h" % mech] + coop

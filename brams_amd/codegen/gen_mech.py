@@ -25,6 +25,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 if HERE not in sys.path:
     sys.path.insert(0, HERE)
 import gen_coop  # noqa: E402
+import gen_qssa  # noqa: E402
 
 PKG = os.path.dirname(HERE)
 MECH = "relacs_tuv"
@@ -264,34 +265,13 @@ def main():
     w("}")
     w("")
 
-    # ---------------- production / loss of the QSSA split
-    def dwexpr(r, s):
-        rs = react[r]
-        if s not in rs:          # negative product (CB07_TUV): dratedc never assigns dw(r,s)
-            return "0.0"
-        if len(rs) == 1:
-            return "rk[%d]" % r
-        o = rs[1] if rs[0] == s else rs[0]
-        return "(rk[%d] * y[%d])" % (r, o)
-
-    w("// QSSA's P - L c split: chem_spack_rates.f90:63-192, chem_spack_dratedc.f90:62-296,")
-    w("// chem_spack_fexprod.f90:64-448, chem_spack_fexloss.f90:64-284.  P: the positive")
-    w("// stoichiometric terms c w_r, L: -c dw_rs over the negative ones (dw_rs = rk_r y_other,")
-    w("// y_s itself in a self-reaction), in reaction order; rows with no term are 0.")
-    w("__device__ __forceinline__ void mech_prod_loss(const double* rk, const double* y, double* P, double* L) {")
+    # operations of QSSA's P - L c split: w_r and the two sums in reaction order
     upos = sorted({r for terms in prod.values() for c, r in terms if c > 0})
-    for r in upos:
-        w("  const double w%d = %s;" % (r, wexpr(r)))
     fl_pl = sum(len(react[r]) for r in upos)
     for s in range(ns):
-        pt = [(c, "w%d" % r) for c, r in prod.get(s, []) if c > 0]
-        lt = [(-c, dwexpr(r, s)) for c, r in prod.get(s, []) if c < 0]
-        w("  P[%d] = %s;" % (s, sum_terms(pt) if pt else "0.0"))
-        w("  L[%d] = %s;" % (s, sum_terms(lt) if lt else "0.0"))
-        fl_pl += nflop_sum_pl([c for c, _ in pt]) + nflop_sum_pl([c for c, _ in lt])
-        fl_pl += sum(1 for _, e in lt if "*" in e)
-    w("}")
-    w("")
+        neg = [(c, r) for c, r in prod.get(s, []) if c < 0]
+        fl_pl += nflop_sum_pl([c for c, _ in prod.get(s, []) if c > 0]) + nflop_sum_pl([c for c, _ in neg])
+        fl_pl += sum(1 for _, r in neg if s in react[r] and len(react[r]) == 2)
 
     def jexpr(i, j):
         terms = []
@@ -455,6 +435,8 @@ def main():
     text = "\n".join(L) + "\n"
     emit_slab(m, ns, react, prod, jt, perm, F, slot, sentries, sidx, wexpr, sum_terms, jexpr, rate_expr)
     emit_coop(m, ns, nr, react, prod, jt, perm, F, sidx, rate_rhs)
+    write(MECH + "_qssa.h", gen_qssa.emit(ns, nr, react, prod, m["reactions"], rate_rhs,
+                                          gen_coop.literal_rates(m["reactions"]), MECH, m["name"]))
     out = os.path.join(GEN, MECH + "_gen.h")
     old = open(out).read() if os.path.exists(out) else None
     if old != text:
@@ -472,8 +454,12 @@ def emit_coop(m, ns, nr, react, prod, jt, perm, F, sidx, rate_rhs):
     rows = place["rows"] or gen_coop.default_rows(mech, place["waves"], place["dense"])
     plan = gen_coop.Plan(mech, place["waves"], place["dense"], rows, place["rk_regs"],
                          gen_coop.literal_rates(m["reactions"]))
-    text = gen_coop.emit(mech, plan, m["reactions"], rate_rhs, MECH, m["name"])
-    out = os.path.join(GEN, MECH + "_coop.h")
+    write(MECH + "_coop.h", gen_coop.emit(mech, plan, m["reactions"], rate_rhs, MECH, m["name"]))
+
+
+def write(name, text):
+    """A generated header, left alone if it is the same already."""
+    out = os.path.join(GEN, name)
     old = open(out).read() if os.path.exists(out) else None
     if old != text:
         with open(out, "w") as fh:

@@ -117,6 +117,26 @@ def test_qssa_accumulates_into_existing_tendency():
     assert nfail == 0
 
 
+@pytest.mark.parametrize("nx,ny,nz,itchim", [(1, 1, 1, 1), (9, 7, 1, 2), (8, 4, 2, 3), (13, 5, 1, 64), (5, 13, 3, 75)])
+def test_qssa_ragged_groups_match_oracle(nx, ny, nz, itchim):
+    """1, 63, 64, 65 and 195 cells, so that the last 64 are partly or wholly
+    there, and sub-step counts of one bit, several and all."""
+    print("case qssa %dx%dx%d itchim=%d" % (nx, ny, nz, itchim), flush=True)
+    grid = Grid(nx, ny, nz)
+    wl = make_workload(grid, seed=nx, sza="random", all_ppbm=True)
+    base = [np.asfortranarray(np.full_like(x, 0.25)) for x in wl["sc_p"]]
+    tend, rc, st, _ = _gpu(wl, itchim, sc_t=base)
+    hs, orc = O.run_oracle_qssa(wl, itchim, sc_t=base)
+    assert rc == 0 and orc == 0 and st.cells == grid.ncell
+    idx = _interior(grid)
+    for s in range(NS):
+        frame = np.ones(tend[s].shape, bool)
+        frame[idx] = False
+        assert np.array_equal(tend[s][frame], base[s][frame])
+    _, nfail = compare(grid, wl, tend, hs)
+    assert nfail == 0
+
+
 def test_qssa_host_entry_matches_device_entry():
     from brams_amd.chem import run_workload_qssa_host
     grid = Grid(12, 9, 7)
