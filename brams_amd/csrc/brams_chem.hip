@@ -69,6 +69,27 @@ struct DevBuf {
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
+// pinned host buffer that only grows: copies from and to it are single
+// transfers, where pageable memory goes through the driver's own buffers with
+// a wait each (about 10 us a copy)
+struct HostBuf {
+  void* p = nullptr;
+  size_t n = 0;
+  hipError_t ensure(size_t bytes) {
+    if (bytes <= n) return hipSuccess;
+    release();
+    hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocDefault);
+    if (e == hipSuccess) n = bytes;
+    return e;
+  }
+  void release() {
+    if (p) hipHostFree(p);
+    p = nullptr;
+    n = 0;
+  }
+  template <class T> T* as() const { return static_cast<T*>(p); }
+};
+
 // Kernel forms of the 64-cell blocks, by the numbers that callers know
 // (brams_chem_set_form).  0..2 were layouts that never ran; 3..5 were register
 // budgets of a one-lane-per-cell kernel.  The cooperative block kernel has one
@@ -88,7 +109,19 @@ struct GridState {
   int m1 = 0, m2 = 0, m3 = 0, ia = 0, iz = 0, ja = 0, jz = 0;
   long long ncell = 0;
   std::vector<int> sizes;        // AllocIndex block sizes
-  DevBuf block_start, mask, attempts, substeps, failed, forced, thresh, order_thresh;
+  DevBuf block_start;
+  // what a step reports, one allocation that one copy brings to the host:
+  // per block attempts, substeps, failed, forced error and threshold pivots,
+  // then the pivots of the ordering and the mask
+  DevBuf status;
+  int* attempts() const { return status.as<int>(); }
+  int* substeps() const { return attempts() + sizes.size(); }
+  int* failed() const { return attempts() + 2 * sizes.size(); }
+  float* forced() const { return (float*)(attempts() + 3 * sizes.size()); }
+  int* thresh() const { return attempts() + 4 * sizes.size(); }
+  int* order_thresh() const { return attempts() + 5 * sizes.size(); }
+  unsigned* mask() const { return (unsigned*)(order_thresh() + 1); }
+  size_t status_bytes() const { return sizeof(int) * (5 * sizes.size() + 1 + MECH_MASK_WORDS); }
   bool blk_hist = false;         // attempts[] holds a previous call on this grid
   long long hist_cells = -1;     // fallback memory of the surrogate step (-1: to be started)
   DevBuf cell_dt;
@@ -105,8 +138,10 @@ struct State {
   int device = 0;
   std::vector<GridState*> grids;
   GridState* cur = nullptr;      // grid of the last call
-  // host-entry staging
-  DevBuf sc_p, sc_t, sc_t_dyn, met, jphoto, last_dt, consts;
+  // host entries: their arrays on the device, and on the way there and back
+  DevBuf host_dev;
+  HostBuf host_pin;
+  HostBuf h_status;              // a grid's status on its way to the host
   // surrogate step
   DevBuf sur_X, sur_out, sur_flag, sur_list, sur_chunk, sur_reason, fb_dt, fb_att, mask_all;
   // work ordering (sched_kernels.h): sort scratch and block order
@@ -125,13 +160,71 @@ struct State {
 };
 State g;
 
-// the host entries' per-species constants in g.consts: weight f32,
-// transport flag i32, atol f64, rtol f64, each region 256-byte aligned
+// the host entries' per-species constants: weight f32, transport flag i32,
+// atol f64, rtol f64, each region 256-byte aligned
 constexpr size_t kConstRound(size_t x) { return (x + 255) / 256 * 256; }
 constexpr size_t kConstOffT = kConstRound(sizeof(float) * MECH_NS);
 constexpr size_t kConstOffA = kConstOffT + kConstRound(sizeof(int) * MECH_NS);
 constexpr size_t kConstOffR = kConstOffA + kConstRound(sizeof(double) * MECH_NS);
 constexpr size_t kConstBytes = kConstOffR + kConstRound(sizeof(double) * MECH_NS);
+
+// The host entries' arrays, side by side in g.host_dev: a host entry has about
+// a hundred of them (47 species, each an array of its own), and a copy of a
+// pageable array costs 10 us whatever its size.  Up to kStageBytes they are
+// packed into pinned memory and cross in one copy each way; above it, where
+// the copies' own time counts and packing would add a pass over the data, each
+// array is copied by itself.  QSSA calls with 0.07 / 2 / 20 / 39 / 97 / 231 MB
+// take 1.09 / 1.10 / 2.3 / 3.2 / 5.8 / 13.2 ms array by array and 0.23 / 0.32 /
+// 1.5 / 2.9 / 7.2 / 16.6 ms packed, so the line lies just below where they meet.
+constexpr size_t kStageBytes = (size_t)32 << 20;
+struct HostArrays {
+  struct Span {
+    void* host;
+    size_t off, bytes;
+  };
+  std::vector<Span> in, out;
+  size_t end = 0;
+  // room for n bytes on the device, filled from src (null: left as it is)
+  size_t add(const void* src, size_t n) {
+    const size_t off = end;
+    if (src) in.push_back({const_cast<void*>(src), off, n});
+    end = (end + n + 255) / 256 * 256;
+    return off;
+  }
+  bool staged() const { return end <= kStageBytes; }
+  int load(hipStream_t st) const {
+    HIP_TRY(g.host_dev.ensure(end));
+    char* d = g.host_dev.as<char>();
+    if (!staged()) {
+      for (const Span& x : in) HIP_TRY(hipMemcpyAsync(d + x.off, x.host, x.bytes, hipMemcpyHostToDevice, st));
+      return 0;
+    }
+    HIP_TRY(g.host_pin.ensure(end));
+    for (const Span& x : in) std::memcpy(g.host_pin.as<char>() + x.off, x.host, x.bytes);
+    HIP_TRY(hipMemcpyAsync(d, g.host_pin.p, end, hipMemcpyHostToDevice, st));
+    return 0;
+  }
+  // the out arrays' copies; they hold their values after a synchronisation of
+  // st and unpack()
+  int fetch(hipStream_t st) const {
+    const char* d = g.host_dev.as<char>();
+    if (!staged()) {
+      for (const Span& x : out) HIP_TRY(hipMemcpyAsync(x.host, d + x.off, x.bytes, hipMemcpyDeviceToHost, st));
+      return 0;
+    }
+    size_t lo = end, hi = 0;
+    for (const Span& x : out) {
+      lo = std::min(lo, x.off);
+      hi = std::max(hi, x.off + x.bytes);
+    }
+    HIP_TRY(hipMemcpyAsync(g.host_pin.as<char>() + lo, d + lo, hi - lo, hipMemcpyDeviceToHost, st));
+    return 0;
+  }
+  void unpack() const {
+    if (staged())
+      for (const Span& x : out) std::memcpy(x.host, g.host_pin.as<char>() + x.off, x.bytes);
+  }
+};
 
 // Bookkeeping of brams_chem_rodas3_dyndt_device_noalloc (block starts, mask
 // words, per-block counters, failure count) lives in one file-scope device
@@ -215,17 +308,10 @@ int ensure_grid(int m1, int m2, int m3, int ia, int iz, int ja, int jz) {
   for (int b = 0; b < nob; ++b) start[b + 1] = start[b] + sizes[b];
   hipError_t e = gs->block_start.ensure(sizeof(int) * (nob + 1));
   if (e == hipSuccess) e = hipMemcpy(gs->block_start.p, start.data(), sizeof(int) * (nob + 1), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = gs->mask.ensure(sizeof(unsigned) * MECH_MASK_WORDS);
-  if (e == hipSuccess) e = gs->attempts.ensure(sizeof(int) * nob);
-  if (e == hipSuccess) e = gs->substeps.ensure(sizeof(int) * nob);
-  if (e == hipSuccess) e = gs->failed.ensure(sizeof(int) * nob);
-  if (e == hipSuccess) e = gs->forced.ensure(sizeof(float) * nob);
-  if (e == hipSuccess) e = gs->thresh.ensure(sizeof(int) * nob);
-  if (e == hipSuccess) e = gs->order_thresh.ensure(sizeof(int));
+  if (e == hipSuccess) e = gs->status.ensure(gs->status_bytes());
   if (e != hipSuccess) {
-    DevBuf* bufs[] = {&gs->block_start, &gs->mask, &gs->attempts, &gs->substeps, &gs->failed,
-                      &gs->forced, &gs->thresh, &gs->order_thresh};
-    for (DevBuf* b : bufs) b->release();
+    gs->block_start.release();
+    gs->status.release();
     delete gs;
     return fail(-100 - (int)e, "grid state allocation failed: %s", hipGetErrorString(e));
   }
@@ -256,7 +342,7 @@ int order_blocks(int b0, int n, hipStream_t st) {
   HIP_TRY(g.sort_ids.ensure(sizeof(int) * n));
   HIP_TRY(g.order.ensure(sizeof(int) * n));
   hipLaunchKernelGGL(brams::block_keys, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                     g.cur->attempts.as<int>(), b0, n, g.sort_keys.as<int>(), g.sort_ids.as<int>());
+                     g.cur->attempts(), b0, n, g.sort_keys.as<int>(), g.sort_ids.as<int>());
   HIP_TRY(hipGetLastError());
   return sort_desc(g.sort_keys.as<int>(), g.sort_ids.as<int>(), n, g.order.as<int>(), st);
 }
@@ -274,13 +360,13 @@ int launch_step(brams::StepParams p, hipStream_t st) {
   GridState& gs = *g.cur;
   const int nob = (int)gs.sizes.size();
   p.block_start = gs.block_start.as<int>();
-  p.mask = gs.mask.as<unsigned>();
-  p.blk_attempts = gs.attempts.as<int>();
-  p.blk_substeps = gs.substeps.as<int>();
-  p.blk_failed = gs.failed.as<int>();
-  p.blk_forced = gs.forced.as<float>();
-  p.blk_thresh = gs.thresh.as<int>();
-  p.order_thresh = gs.order_thresh.as<int>();
+  p.mask = gs.mask();
+  p.blk_attempts = gs.attempts();
+  p.blk_substeps = gs.substeps();
+  p.blk_failed = gs.failed();
+  p.blk_forced = gs.forced();
+  p.blk_thresh = gs.thresh();
+  p.order_thresh = gs.order_thresh();
   const std::vector<int>& sz = gs.sizes;
   int nbig = 0;
   while (nbig < nob && sz[nbig] > 64) ++nbig;
@@ -335,15 +421,15 @@ int launch_ros2_step(brams::StepParams p, hipStream_t st) {
   GridState& gs = *g.cur;
   const int nob = (int)gs.sizes.size();
   p.block_start = gs.block_start.as<int>();
-  p.mask = gs.mask.as<unsigned>();
-  p.blk_attempts = gs.attempts.as<int>();
-  p.blk_substeps = gs.substeps.as<int>();
-  p.blk_failed = gs.failed.as<int>();
-  p.blk_forced = gs.forced.as<float>();
-  p.blk_thresh = gs.thresh.as<int>();
+  p.mask = gs.mask();
+  p.blk_attempts = gs.attempts();
+  p.blk_substeps = gs.substeps();
+  p.blk_failed = gs.failed();
+  p.blk_forced = gs.forced();
+  p.blk_thresh = gs.thresh();
   p.order_thresh = nullptr;
-  HIP_TRY(hipMemcpyAsync(gs.mask.p, kStructMask.w, sizeof kStructMask.w, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemsetAsync(gs.order_thresh.p, 0, sizeof(int), st));
+  HIP_TRY(hipMemcpyAsync(gs.mask(), kStructMask.w, sizeof kStructMask.w, hipMemcpyHostToDevice, st));
+  HIP_TRY(hipMemsetAsync(gs.order_thresh(), 0, sizeof(int), st));
   int nbig = 0;
   while (nbig < nob && gs.sizes[nbig] > 64) ++nbig;
   // ROS2 never had a form 4
@@ -377,21 +463,18 @@ int launch_ros2_step(brams::StepParams p, hipStream_t st) {
 int collect_stats(hipStream_t st) {
   GridState& gs = *g.cur;
   const int nob = (int)gs.sizes.size();
+  HIP_TRY(g.h_status.ensure(gs.status_bytes()));
+  HIP_TRY(hipMemcpyAsync(g.h_status.p, gs.status.p, gs.status_bytes(), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  gs.h_att.resize(nob);
-  gs.h_sub.resize(nob);
-  gs.h_fail.resize(nob);
-  gs.h_forced.resize(nob);
-  gs.h_thresh.resize(nob);
-  unsigned mw[MECH_MASK_WORDS];
-  int order_viol = 0;
-  HIP_TRY(hipMemcpy(gs.h_att.data(), gs.attempts.p, sizeof(int) * nob, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(gs.h_sub.data(), gs.substeps.p, sizeof(int) * nob, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(gs.h_fail.data(), gs.failed.p, sizeof(int) * nob, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(gs.h_forced.data(), gs.forced.p, sizeof(float) * nob, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(gs.h_thresh.data(), gs.thresh.p, sizeof(int) * nob, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(&order_viol, gs.order_thresh.p, sizeof(int), hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(mw, gs.mask.p, sizeof mw, hipMemcpyDeviceToHost));
+  const int* h = g.h_status.as<int>();
+  const float* hf = (const float*)(h + 3 * nob);
+  gs.h_att.assign(h, h + nob);
+  gs.h_sub.assign(h + nob, h + 2 * nob);
+  gs.h_fail.assign(h + 2 * nob, h + 3 * nob);
+  gs.h_forced.assign(hf, hf + nob);
+  gs.h_thresh.assign(h + 4 * nob, h + 5 * nob);
+  const int order_viol = h[5 * nob];
+  const unsigned* mw = (const unsigned*)(h + 5 * nob + 1);
   brams_chem_stats s{};
   s.cells = gs.ncell;
   s.blocks = nob;
@@ -798,13 +881,13 @@ int brams_chem_rodas3_dyndt_device_grids(const brams_chem_dev_args* a, int32_t n
     brams::StepParams& p = ps[i];
     fill_params(&a[i], p);
     p.block_start = gs->block_start.as<int>();
-    p.mask = gs->mask.as<unsigned>();
-    p.blk_attempts = gs->attempts.as<int>();
-    p.blk_substeps = gs->substeps.as<int>();
-    p.blk_failed = gs->failed.as<int>();
-    p.blk_forced = gs->forced.as<float>();
-    p.blk_thresh = gs->thresh.as<int>();
-    p.order_thresh = gs->order_thresh.as<int>();
+    p.mask = gs->mask();
+    p.blk_attempts = gs->attempts();
+    p.blk_substeps = gs->substeps();
+    p.blk_failed = gs->failed();
+    p.blk_forced = gs->forced();
+    p.blk_thresh = gs->thresh();
+    p.order_thresh = gs->order_thresh();
     const int tag = i << brams::kGridShift;
     int nbig = 0;
     while (nbig < nob && gs->sizes[nbig] > 64) ++nbig;
@@ -1176,41 +1259,35 @@ int host_step(const brams_chem_args* a, int solver) {
 
   const long long n3d = (long long)a->m1 * a->m2 * a->m3;
   const size_t fsz = sizeof(float) * n3d;
-  HIP_TRY(g.sc_p.ensure(fsz * MECH_NS));
-  HIP_TRY(g.met.ensure(fsz * 4));
-  HIP_TRY(g.jphoto.ensure(sizeof(double) * MECH_NPHOT * n3d));
-  HIP_TRY(g.last_dt.ensure(sizeof(double) * nob));
   // consts: weight[MECH_NS] f32 | transported[MECH_NS] i32 | atol[MECH_NS] f64 | rtol[MECH_NS] f64
   const size_t coff_w = 0, coff_t = kConstOffT, coff_a = kConstOffA, coff_r = kConstOffR;
-  HIP_TRY(g.consts.ensure(kConstBytes));
-  if (need_t) HIP_TRY(g.sc_t.ensure(fsz * MECH_NS));
-  if (need_td) HIP_TRY(g.sc_t_dyn.ensure(fsz * MECH_NS));
-  hipStream_t st = nullptr;
-  char* sc = g.sc_p.as<char>();
-  for (int s = 0; s < MECH_NS; ++s)
-    HIP_TRY(hipMemcpyAsync(sc + s * fsz, a->sc_p[s], fsz, hipMemcpyHostToDevice, st));
-  if (need_t)
-    for (int s = 0; s < MECH_NS; ++s)
-      HIP_TRY(hipMemcpyAsync(g.sc_t.as<char>() + s * fsz, a->sc_t[s], fsz, hipMemcpyHostToDevice, st));
-  if (need_td)
-    for (int s = 0; s < MECH_NS; ++s)
-      HIP_TRY(hipMemcpyAsync(g.sc_t_dyn.as<char>() + s * fsz, a->sc_t_dyn[s], fsz,
-                             hipMemcpyHostToDevice, st));
-  char* met = g.met.as<char>();
-  HIP_TRY(hipMemcpyAsync(met + 0 * fsz, a->pp, fsz, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(met + 1 * fsz, a->pi0, fsz, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(met + 2 * fsz, a->theta, fsz, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(met + 3 * fsz, a->rv, fsz, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(g.jphoto.p, a->jphoto, sizeof(double) * MECH_NPHOT * n3d,
-                         hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(g.last_dt.p, a->last_accepted_dt, sizeof(double) * nob,
-                         hipMemcpyHostToDevice, st));
-  char cbuf[kConstBytes];
+  char cbuf[kConstBytes] = {};
   std::memcpy(cbuf + coff_w, a->weight, sizeof(float) * MECH_NS);
   std::memcpy(cbuf + coff_t, flags, sizeof(int) * MECH_NS);
   std::memcpy(cbuf + coff_a, a->atol, sizeof(double) * MECH_NS);
   std::memcpy(cbuf + coff_r, a->rtol, sizeof(double) * MECH_NS);
-  HIP_TRY(hipMemcpy(g.consts.p, cbuf, sizeof cbuf, hipMemcpyHostToDevice));
+  HostArrays h;
+  const size_t o_consts = h.add(cbuf, sizeof cbuf);
+  const size_t o_pp = h.add(a->pp, fsz), o_pi0 = h.add(a->pi0, fsz);
+  const size_t o_theta = h.add(a->theta, fsz), o_rv = h.add(a->rv, fsz);
+  const size_t o_jphoto = h.add(a->jphoto, sizeof(double) * MECH_NPHOT * n3d);
+  // the species are one array on the device, so a gap follows the last only
+  const auto species = [&](const auto* x) {
+    const size_t off = h.end;
+    for (int s = 0; s < MECH_NS; ++s) h.in.push_back({const_cast<float*>(x[s]), off + s * fsz, fsz});
+    h.add(nullptr, fsz * MECH_NS);
+    return off;
+  };
+  const size_t o_td = need_td ? species(a->sc_t_dyn) : 0;
+  const size_t o_p = species(a->sc_p);
+  const size_t o_dt = h.add(a->last_accepted_dt, sizeof(double) * nob);
+  const size_t o_t = need_t ? species(a->sc_t) : 0;
+  for (int s = 0; s < MECH_NS; ++s)
+    h.out.push_back({need_t ? a->sc_t[s] : a->sc_p[s], (need_t ? o_t : o_p) + s * fsz, fsz});
+  h.out.push_back({a->last_accepted_dt, o_dt, sizeof(double) * nob});
+  hipStream_t st = nullptr;
+  if ((rc = h.load(st))) return rc;
+  char* d = g.host_dev.as<char>();
 
   brams::StepParams p{};
   p.m1 = a->m1; p.m2 = a->m2; p.m3 = a->m3;
@@ -1218,32 +1295,25 @@ int host_step(const brams_chem_args* a, int solver) {
   p.nk = a->m1 - 2; p.ni = a->iz - a->ia + 1;
   p.dtlt = a->dtlt; p.ndyn = a->n_dyn_chem; p.split = a->split_method;
   p.cp = a->cp; p.cpor = a->cpor; p.p00 = a->p00;
-  p.pp = (const float*)(met + 0 * fsz);
-  p.pi0 = (const float*)(met + 1 * fsz);
-  p.theta = (const float*)(met + 2 * fsz);
-  p.rv = (const float*)(met + 3 * fsz);
-  p.jphoto = g.jphoto.as<double>();
-  p.weight = (const float*)(g.consts.as<char>() + coff_w);
-  p.transported = (const int*)(g.consts.as<char>() + coff_t);
-  p.atol = (const double*)(g.consts.as<char>() + coff_a);
-  p.rtol = (const double*)(g.consts.as<char>() + coff_r);
-  p.sc_p = g.sc_p.as<float>();
-  p.sc_t = need_t ? g.sc_t.as<float>() : nullptr;
-  p.sc_t_dyn = need_td ? g.sc_t_dyn.as<float>() : nullptr;
+  p.pp = (const float*)(d + o_pp);
+  p.pi0 = (const float*)(d + o_pi0);
+  p.theta = (const float*)(d + o_theta);
+  p.rv = (const float*)(d + o_rv);
+  p.jphoto = (const double*)(d + o_jphoto);
+  p.weight = (const float*)(d + o_consts + coff_w);
+  p.transported = (const int*)(d + o_consts + coff_t);
+  p.atol = (const double*)(d + o_consts + coff_a);
+  p.rtol = (const double*)(d + o_consts + coff_r);
+  p.sc_p = (float*)(d + o_p);
+  p.sc_t = need_t ? (float*)(d + o_t) : nullptr;
+  p.sc_t_dyn = need_td ? (float*)(d + o_td) : nullptr;
   p.n3d = n3d;
-  p.last_dt = g.last_dt.as<double>();
+  p.last_dt = (double*)(d + o_dt);
   if ((rc = solver == brams::kRos2 ? launch_ros2_step(p, st) : launch_step(p, st))) return rc;
   // results back into the caller's arrays
-  if (need_t) {
-    for (int s = 0; s < MECH_NS; ++s)
-      HIP_TRY(hipMemcpyAsync(a->sc_t[s], g.sc_t.as<char>() + s * fsz, fsz, hipMemcpyDeviceToHost, st));
-  } else {
-    for (int s = 0; s < MECH_NS; ++s)
-      HIP_TRY(hipMemcpyAsync(a->sc_p[s], sc + s * fsz, fsz, hipMemcpyDeviceToHost, st));
-  }
-  HIP_TRY(hipMemcpyAsync(a->last_accepted_dt, g.last_dt.p, sizeof(double) * nob,
-                         hipMemcpyDeviceToHost, st));
-  return collect_stats(st);
+  if ((rc = h.fetch(st))) return rc;
+  if ((rc = collect_stats(st)) >= 0) h.unpack();
+  return rc;
 }
 
 // One QSSA step (chem_qssa) on device arrays already in p: the counter is
@@ -1309,46 +1379,41 @@ int brams_chem_qssa(const brams_chem_args* a, int32_t itchim) {
   if (!g.init && (rc = brams_chem_init(0))) return rc;
   const long long n3d = (long long)a->m1 * a->m2 * a->m3;
   const size_t fsz = sizeof(float) * n3d;
-  HIP_TRY(g.sc_p.ensure(fsz * MECH_NS));
-  HIP_TRY(g.sc_t.ensure(fsz * MECH_NS));
-  HIP_TRY(g.met.ensure(fsz * 4));
-  HIP_TRY(g.jphoto.ensure(sizeof(double) * MECH_NPHOT * n3d));
-  HIP_TRY(g.consts.ensure(kConstBytes));
-  hipStream_t st = nullptr;
-  char* sc = g.sc_p.as<char>();
-  char* tc = g.sc_t.as<char>();
+  HostArrays h;
+  const size_t o_weight = h.add(a->weight, sizeof(float) * MECH_NS);
+  const size_t o_pp = h.add(a->pp, fsz), o_pi0 = h.add(a->pi0, fsz);
+  const size_t o_theta = h.add(a->theta, fsz), o_rv = h.add(a->rv, fsz);
+  const size_t o_jphoto = h.add(a->jphoto, sizeof(double) * MECH_NPHOT * n3d);
+  const size_t o_p = h.add(nullptr, fsz * MECH_NS), o_t = h.add(nullptr, fsz * MECH_NS);
   for (int s = 0; s < MECH_NS; ++s) {
-    HIP_TRY(hipMemcpyAsync(sc + s * fsz, a->sc_p[s], fsz, hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(tc + s * fsz, a->sc_t[s], fsz, hipMemcpyHostToDevice, st));
+    h.in.push_back({a->sc_p[s], o_p + s * fsz, fsz});
+    h.in.push_back({a->sc_t[s], o_t + s * fsz, fsz});
+    h.out.push_back({a->sc_t[s], o_t + s * fsz, fsz});
   }
-  char* met = g.met.as<char>();
-  HIP_TRY(hipMemcpyAsync(met + 0 * fsz, a->pp, fsz, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(met + 1 * fsz, a->pi0, fsz, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(met + 2 * fsz, a->theta, fsz, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(met + 3 * fsz, a->rv, fsz, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(g.jphoto.p, a->jphoto, sizeof(double) * MECH_NPHOT * n3d, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpy(g.consts.p, a->weight, sizeof(float) * MECH_NS, hipMemcpyHostToDevice));
+  hipStream_t st = nullptr;
+  if ((rc = h.load(st))) return rc;
+  char* d = g.host_dev.as<char>();
   brams::StepParams p{};
   p.m1 = a->m1; p.m2 = a->m2; p.m3 = a->m3;
   p.ia = a->ia; p.iz = a->iz; p.ja = a->ja; p.jz = a->jz;
   p.nk = a->m1 - 2; p.ni = a->iz - a->ia + 1;
   p.dtlt = a->dtlt;
   p.cp = a->cp; p.cpor = a->cpor; p.p00 = a->p00;
-  p.pp = (const float*)(met + 0 * fsz);
-  p.pi0 = (const float*)(met + 1 * fsz);
-  p.theta = (const float*)(met + 2 * fsz);
-  p.rv = (const float*)(met + 3 * fsz);
-  p.jphoto = g.jphoto.as<double>();
-  p.weight = g.consts.as<float>();
-  p.sc_p = g.sc_p.as<float>();
-  p.sc_t = g.sc_t.as<float>();
+  p.pp = (const float*)(d + o_pp);
+  p.pi0 = (const float*)(d + o_pi0);
+  p.theta = (const float*)(d + o_theta);
+  p.rv = (const float*)(d + o_rv);
+  p.jphoto = (const double*)(d + o_jphoto);
+  p.weight = (const float*)(d + o_weight);
+  p.sc_p = (float*)(d + o_p);
+  p.sc_t = (float*)(d + o_t);
   p.n3d = n3d;
   const long long ncell = (long long)(a->m1 - 2) * (a->iz - a->ia + 1) * (a->jz - a->ja + 1);
   const int nfatal = qssa_step(p, itchim, ncell, st);
   if (nfatal < 0) return nfatal;
-  for (int s = 0; s < MECH_NS; ++s)
-    HIP_TRY(hipMemcpyAsync(a->sc_t[s], tc + s * fsz, fsz, hipMemcpyDeviceToHost, st));
+  if ((rc = h.fetch(st))) return rc;
   HIP_TRY(hipStreamSynchronize(st));
+  h.unpack();
   return nfatal;
 }
 
@@ -1437,15 +1502,15 @@ const char* brams_chem_last_error(void) { return g_err.c_str(); }
 
 void brams_chem_finalize(void) {
   for (GridState* gs : g.grids) {
-    DevBuf* gb[] = {&gs->block_start, &gs->mask, &gs->attempts, &gs->substeps, &gs->failed,
-                    &gs->forced, &gs->thresh, &gs->order_thresh, &gs->cell_dt};
+    DevBuf* gb[] = {&gs->block_start, &gs->status, &gs->cell_dt};
     for (DevBuf* b : gb) b->release();
     delete gs;
   }
   g.grids.clear();
   g.cur = nullptr;
-  DevBuf* bufs[] = {&g.sc_p, &g.sc_t, &g.sc_t_dyn, &g.met, &g.jphoto, &g.last_dt, &g.consts,
-                    &g.sur_X, &g.sur_out, &g.sur_flag, &g.sur_list, &g.sur_chunk,
+  g.host_pin.release();
+  g.h_status.release();
+  DevBuf* bufs[] = {&g.host_dev, &g.sur_X, &g.sur_out, &g.sur_flag, &g.sur_list, &g.sur_chunk,
                     &g.sur_reason, &g.fb_dt, &g.fb_att, &g.mask_all, &g.sort_keys, &g.sort_ids,
                     &g.sort_count, &g.sort_off, &g.order, &g.half_y};
   for (DevBuf* b : bufs) b->release();

@@ -148,6 +148,18 @@ def test_qssa_host_entry_matches_device_entry():
         assert np.array_equal(a, b)
 
 
+def test_qssa_host_entry_above_the_staging_size_matches_device_entry():
+    """40x40x40: 39 MB of arrays, each copied by itself."""
+    from brams_amd.chem import run_workload_qssa_host
+    grid = Grid(40, 40, 40)
+    wl = make_workload(grid, seed=4, all_ppbm=True)
+    host, rc = run_workload_qssa_host(wl)
+    tend, rc2, _, _ = _gpu(wl)
+    assert rc == 0 and rc2 == 0
+    for a, b in zip(host, tend):
+        assert np.array_equal(a, b)
+
+
 def test_qssa_cell_reaching_1e20_is_counted_and_keeps_its_tendency():
     print("case qssa 1e20 cell, 5x4x3", flush=True)
     grid = Grid(5, 4, 3)
