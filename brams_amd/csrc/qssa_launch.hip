@@ -162,12 +162,12 @@ static_assert(MECH_QSSA_SLOTS <= 320 && kQssaLds <= 160 * 1024, "the exchange fi
 static_assert(MECH_QSSA_WAVES * 64 >= MECH_NS, "one thread per weight");
 
 __global__ __launch_bounds__(MECH_QSSA_WAVES * 64, kQssaWaves) void qssa_cells(StepParams p, int itchim, long long ncell,
-                                                                              int* nfatal) {
+                                                                              long long first, int* nfatal) {
   __shared__ double lds[MECH_QSSA_SLOTS * 64];
   __shared__ double2 weight[MECH_NS];
   __shared__ int fatal[64];
   const int lane = threadIdx.x & 63;
-  const long long c = (long long)blockIdx.x * 64 + lane;
+  const long long c = first + (long long)blockIdx.x * 64 + lane;
   const long long g = c < ncell ? c : ncell - 1;
   const int k = 1 + (int)(g % p.nk);
   const long long t = g / p.nk;
@@ -186,9 +186,13 @@ __global__ __launch_bounds__(MECH_QSSA_WAVES * 64, kQssaWaves) void qssa_cells(S
 }
 
 hipError_t launch_qssa(const StepParams& p, int itchim, long long ncell, int* nfatal, hipStream_t st) {
-  if (ncell <= 0) return hipSuccess;
-  hipLaunchKernelGGL(qssa_cells, dim3((unsigned)((ncell + 63) / 64)), dim3(MECH_QSSA_WAVES * 64), 0, st, p, itchim, ncell,
-                     nfatal);
+  // a dispatch counts its work-items in 32 bits: at most 2^31 of them
+  constexpr long long kCells = (1ll << 31) / (MECH_QSSA_WAVES * 64) * 64;
+  for (long long first = 0; first < ncell; first += kCells) {
+    const long long n = ncell - first < kCells ? ncell - first : kCells;
+    hipLaunchKernelGGL(qssa_cells, dim3((unsigned)((n + 63) / 64)), dim3(MECH_QSSA_WAVES * 64), 0, st, p, itchim, ncell,
+                       first, nfatal);
+  }
   return hipGetLastError();
 }
 

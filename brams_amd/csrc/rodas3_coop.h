@@ -392,4 +392,33 @@ __global__ __launch_bounds__(kCoopLanes, MECH_COOP_WAVES / 4) void coop_grids(co
   coop_block<kRodas3, DYN, COUNT>(grids[w >> kGridShift], w & kGridBlockMask, (int)blockIdx.x);
 }
 
+#ifdef __HIPCC__
+// A dispatch counts its work-items in 32 bits, which 8M blocks exceed, so it
+// takes at most half of that many.
+constexpr unsigned kCoopMaxBlocks = 1u << 22;
+
+template <int SOLVER, bool DYN, bool COUNT>
+hipError_t coop_launch(unsigned nblocks, StepParams p, int block0, hipStream_t st) {
+  while (nblocks > 0) {
+    const unsigned n = nblocks < kCoopMaxBlocks ? nblocks : kCoopMaxBlocks;
+    hipLaunchKernelGGL((coop_blocks<SOLVER, DYN, COUNT>), dim3(n), dim3(kCoopLanes), 0, st, p, block0);
+    if (p.block_order) p.block_order += n;
+    block0 += (int)n;
+    nblocks -= n;
+  }
+  return hipGetLastError();
+}
+
+template <bool DYN, bool COUNT>
+hipError_t coop_launch_grids(unsigned nwork, const StepParams* grids, const int* work, hipStream_t st) {
+  while (nwork > 0) {
+    const unsigned n = nwork < kCoopMaxBlocks ? nwork : kCoopMaxBlocks;
+    hipLaunchKernelGGL((coop_grids<DYN, COUNT>), dim3(n), dim3(kCoopLanes), 0, st, grids, work);
+    work += n;
+    nwork -= n;
+  }
+  return hipGetLastError();
+}
+#endif
+
 }  // namespace brams

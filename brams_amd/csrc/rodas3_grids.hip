@@ -18,13 +18,9 @@ hipError_t launch_rodas3_grids(bool first, bool big, unsigned nwork, const StepP
   (void)first, (void)big, (void)st;
   return hipErrorInvalidValue;
 #else
-  if (first)
-    hipLaunchKernelGGL((coop_grids<true, true>), dim3(nwork), dim3(kCoopLanes), 0, st, grids, work);
-  else if (big)
-    hipLaunchKernelGGL((coop_grids<false, true>), dim3(nwork), dim3(kCoopLanes), 0, st, grids, work);
-  else
-    hipLaunchKernelGGL((coop_grids<false, false>), dim3(nwork), dim3(kCoopLanes), 0, st, grids, work);
-  return hipGetLastError();
+  if (first) return coop_launch_grids<true, true>(nwork, grids, work, st);
+  if (big) return coop_launch_grids<false, true>(nwork, grids, work, st);
+  return coop_launch_grids<false, false>(nwork, grids, work, st);
 #endif
 }
 

@@ -13,15 +13,15 @@ namespace brams {
 hipError_t launch_rodas3(unsigned nblocks, const StepParams& p, int block0, hipStream_t st) {
   if (nblocks == 0) return hipSuccess;
 #ifdef BRAMS_MECH_COOP
-  hipLaunchKernelGGL((coop_blocks<kRodas3, false, false>), dim3(nblocks), dim3(kCoopLanes), 0, st, p, block0);
+  return coop_launch<kRodas3, false, false>(nblocks, p, block0, st);
 #else
   if (p.cell_list) return hipErrorInvalidValue;
   if (nblocks >= kLaneManyBlocks)
     hipLaunchKernelGGL((rodas3_blocks<64, false, kLaneManyWaves>), dim3(nblocks), dim3(64), 0, st, p, block0);
   else
     hipLaunchKernelGGL((rodas3_blocks<64, false, 1>), dim3(nblocks), dim3(64), 0, st, p, block0);
-#endif
   return hipGetLastError();
+#endif
 }
 
 }  // namespace brams

@@ -13,14 +13,14 @@ namespace brams {
 hipError_t launch_ros2(unsigned nblocks, const StepParams& p, int block0, hipStream_t st) {
   if (nblocks == 0) return hipSuccess;
 #ifdef BRAMS_MECH_COOP
-  hipLaunchKernelGGL((coop_blocks<kRos2, false, false>), dim3(nblocks), dim3(kCoopLanes), 0, st, p, block0);
+  return coop_launch<kRos2, false, false>(nblocks, p, block0, st);
 #else
   if (nblocks >= kLaneManyBlocks)
     hipLaunchKernelGGL((ros2_blocks<64, kLaneManyWaves>), dim3(nblocks), dim3(64), 0, st, p, block0);
   else
     hipLaunchKernelGGL((ros2_blocks<64, 1>), dim3(nblocks), dim3(64), 0, st, p, block0);
-#endif
   return hipGetLastError();
+#endif
 }
 
 hipError_t launch_ros2_big(unsigned nblocks, const StepParams& p, int block0, hipStream_t st) {
