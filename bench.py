@@ -90,18 +90,20 @@ def qssa_flop_model(itchim):
     """Algorithmic FP64 FLOP of one QSSA call per cell (chem_spack_qssa.f90):
     the rate coefficients and conversions (as RODAS3's per-call term), the
     P/L split, per species the setup (ybid, P/ybid, the exponent) and the
-    tendency (10), and per species and sub-step one subtraction and one FMA."""
+    tendency (10), and per species the itchim sub-steps as a power by repeated
+    squaring (one product a bit, one a set bit, one subtraction and one FMA)."""
     f, ns = mech_flops()
     f_call, _, _ = flop_model()
-    return f_call + f["prod_loss"] + 10 * ns + 3 * ns * itchim
+    power = itchim.bit_length() - 1 + bin(itchim).count("1") + 3
+    return f_call + f["prod_loss"] + (10 + power) * ns
 
 
 # PMC-measured HBM bytes per cell of qssa_cells (read + written),
-# profiles/qssa_kernel_stats_and_traffic.md
-QSSA_TRAFFIC_PER_CELL = 881 + 289
-# the same for tuv_map_interior, bytes per interior grid point at kj 80, kz
-# 125 with 17 reactions mapped (profiles/tuv_jphoto_mapping.md)
-TUV_TRAFFIC_PER_POINT = 254
+# profiles/kernel_stats_and_traffic.md
+QSSA_TRAFFIC_PER_CELL = 750 + 221
+# the same for tuv_map, bytes per interior grid point at kj 80, kz
+# 125 with 17 reactions mapped (profiles/kernel_stats_and_traffic.md)
+TUV_TRAFFIC_PER_POINT = 263
 
 
 MLP_FLOP_PER_CELL = 3 * 2 * (68 * 256 + 3 * 256 * 256 + 256 * 47)
@@ -518,7 +520,7 @@ def bench_tuv(args):
                                % (args.nx, args.ny, args.nz), "points": npts},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": 8000.0, "unit": "GB/s",
                      "frac": achieved / 8000.0, "traffic": TUV_TRAFFIC_PER_POINT * npts,
-                     "kernel": "tuv_map_interior",
+                     "kernel": "tuv_map",
                      "avg_ms": kms / K, "algorithmic_bytes": algo},
     }
     print(json.dumps(line), flush=True)
@@ -749,7 +751,7 @@ def main():
                 "unit": dominant["unit"], "frac": dominant["frac"], "traffic": dominant["traffic"],
                 "algorithmic_bytes": dominant["algorithmic_bytes"],
                 "traffic_note": "HBM bytes per launch: PMC-measured bytes per cell-attempt (RODAS3) or per "
-                                "cell (MLP) x this run's counts, profiles/rodas3_hbm_traffic_pmc.md; "
+                                "cell (MLP) x this run's counts (profiles/); "
                                 "null where that kernel form was not measured",
                 "kernel": dominant["kernel"], "avg_ms": dominant["avg_ms"],
                 "peak_note": "FP64 vector for the RODAS3 kernels (no MFMA issued; MI355X FP64 vector "

@@ -192,7 +192,8 @@ def set_form(form):
 
 
 def tuning():
-    """(chosen form of the current grid, autotuner timings in ms per form)."""
+    """(kernel form of the current grid, ms of its first call's 64-cell blocks
+    per built form: they are one kernel)."""
     import numpy as np
     f = np.zeros(1, np.int32)
     ms = np.zeros(8, np.float32)
