@@ -1,4 +1,4 @@
-// Host entry of the slab kernels (defined in rodas3_slab.hip).
+// The slab layout's parameters and launch interface (no library builds it).
 #pragma once
 #include <hip/hip_runtime.h>
 
