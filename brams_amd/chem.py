@@ -3,8 +3,9 @@
 chem_rodas3_dyndt() keeps the argument names, meaning and units of
 mod_chem_spack_rodas3_dyndt::chem_rodas3_dyndt
 (src/brams/ccatt/chem_spack_rodas3_dyndt.f90:41-131) for the arguments the
-RELACS_TUV path reads; it updates chem1_sc_p (or sc_t) and last_accepted_dt in
-place like the Fortran routine.  chem_ros_dyndt() is the same for the ROS2
+RELACS_TUV path reads; it updates chem1_sc_p (of the transported species sc_t
+instead, with PARALLEL and N_DYN_CHEM=1) and last_accepted_dt in place like the
+Fortran routine.  chem_ros_dyndt() is the same for the ROS2
 solver (chem_spack_ros_dyndt.f90:39-45, CHEMISTRY=3), and chem_qssa() for
 the QSSA solver (chem_spack_qssa.f90:37-43, CHEMISTRY=1), which adds every
 species' tendency to sc_t.  DeviceStep runs any of them on arrays that

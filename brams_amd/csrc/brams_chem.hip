@@ -1282,8 +1282,12 @@ int host_step(const brams_chem_args* a, int solver) {
   const size_t o_p = species(a->sc_p);
   const size_t o_dt = h.add(a->last_accepted_dt, sizeof(double) * nob);
   const size_t o_t = need_t ? species(a->sc_t) : 0;
-  for (int s = 0; s < MECH_NS; ++s)
-    h.out.push_back({need_t ? a->sc_t[s] : a->sc_p[s], (need_t ? o_t : o_p) + s * fsz, fsz});
+  // a PARALLEL step with N_DYN_CHEM=1 writes the transported species' sc_t and
+  // the others' sc_p (rodas3:713-798)
+  for (int s = 0; s < MECH_NS; ++s) {
+    if (need_t) h.out.push_back({a->sc_t[s], o_t + s * fsz, fsz});
+    if (!need_t || !flags[s]) h.out.push_back({a->sc_p[s], o_p + s * fsz, fsz});
+  }
   h.out.push_back({a->last_accepted_dt, o_dt, sizeof(double) * nob});
   hipStream_t st = nullptr;
   if ((rc = h.load(st))) return rc;

@@ -134,8 +134,9 @@ int brams_chem_init(int device);
 /*
  * Drop-in for chem_rodas3_dyndt (chem_spack_rodas3_dyndt.f90:41): integrate
  * every interior cell of one grid over dtlt*N_DYN_CHEM with RODAS3, updating
- * sc_p (or sc_t), last_accepted_dt in place.  Host arrays; the library copies
- * them to and from the device.
+ * sc_p and last_accepted_dt in place; with PARALLEL and N_DYN_CHEM=1 the
+ * transported species' sc_t instead of their sc_p.  Host arrays; the library
+ * copies them to and from the device.
  */
 int brams_chem_rodas3_dyndt(const brams_chem_args *args);
 

@@ -309,7 +309,8 @@ def test_step_untouched_outside_interior_and_constant_species():
 
 
 def test_parallel_split_tendency_identity():
-    """PARALLEL, N_DYN_CHEM=1 adds (new - old)/dtlt to sc_t and leaves sc_p."""
+    """PARALLEL, N_DYN_CHEM=1 adds (new - old)/dtlt to sc_t and leaves sc_p of
+    the transported species."""
     wl = make_workload(Grid(8, 8, 6), seed=4)
     atol, rtol = tolerances("reference")
     hsym, _, _, _ = O.run_oracle(wl, atol, rtol, split_method=0)
