@@ -1220,16 +1220,26 @@ namespace {
 // one chemistry step with host arrays (chem_rodas3_dyndt / chem_ros_dyndt)
 int host_step(const brams_chem_args* a, int solver) {
   if (!a) return fail(-2, "null args");
-  if (!g.init) {
-    int rc = brams_chem_init(0);
-    if (rc) return rc;
-  }
   int rc = check_common(a->m1, a->m2, a->m3, a->ia, a->iz, a->ja, a->jz, a->n_dyn_chem,
                         a->split_method, a->photoj_method, a->dtlt);
   if (rc) return rc;
   if (a->nspecies != MECH_NS || a->nr != MECH_NR || a->nr_photo != MECH_NPHOT)
     return fail(-2, "mechanism sizes %d/%d/%d differ from this library's %s %d/%d/%d", a->nspecies, a->nr,
                 a->nr_photo, MECH_NAME, MECH_NS, MECH_NR, MECH_NPHOT);
+  const bool need_t = a->split_method == BRAMS_SPLIT_PARALLEL && a->n_dyn_chem == 1;
+  const bool need_td = a->split_method == BRAMS_SPLIT_PARALLEL && a->n_dyn_chem > 1;
+  if (need_t && !a->sc_t) return fail(-2, "PARALLEL with N_DYN_CHEM=1 needs sc_t");
+  if (need_td && !a->sc_t_dyn) return fail(-2, "PARALLEL with N_DYN_CHEM>1 needs sc_t_dyn");
+  // every array is read on the host before the device sees it
+  if (!a->pp || !a->pi0 || !a->theta || !a->rv || !a->jphoto || !a->weight || !a->sc_p || !a->block_end ||
+      !a->last_accepted_dt || !a->atol || !a->rtol || (a->n_transported > 0 && !a->transp_chem_index) ||
+      (a->n_not_transported > 0 && !a->no_transp_chem_index))
+    return fail(-2, "null argument (a step needs pp, pi0, theta, rv, jphoto, weight, the transport lists, sc_p, "
+                "block_end, last_accepted_dt, atol, rtol)");
+  for (int s = 0; s < MECH_NS; ++s)
+    if (!a->sc_p[s] || (need_t && !a->sc_t[s]) || (need_td && !a->sc_t_dyn[s]))
+      return fail(-2, "species %d has no sc_p%s array", s + 1, need_t ? " or sc_t" : need_td ? " or sc_t_dyn" : "");
+  if (!g.init && (rc = brams_chem_init(0))) return rc;
   if ((rc = ensure_grid(a->m1, a->m2, a->m3, a->ia, a->iz, a->ja, a->jz))) return rc;
   const int nob = (int)g.cur->sizes.size();
   if (a->nob != nob) return fail(-2, "nob %d does not match the AllocIndex partition (%d)", a->nob, nob);
@@ -1252,10 +1262,6 @@ int host_step(const brams_chem_args* a, int solver) {
   }
   for (int s = 0; s < MECH_NS; ++s)
     if (flags[s] < 0) return fail(-2, "species %d in neither transport list", s + 1);
-  const bool need_t = a->split_method == BRAMS_SPLIT_PARALLEL && a->n_dyn_chem == 1;
-  const bool need_td = a->split_method == BRAMS_SPLIT_PARALLEL && a->n_dyn_chem > 1;
-  if (need_t && !a->sc_t) return fail(-2, "PARALLEL with N_DYN_CHEM=1 needs sc_t");
-  if (need_td && !a->sc_t_dyn) return fail(-2, "PARALLEL with N_DYN_CHEM>1 needs sc_t_dyn");
 
   const long long n3d = (long long)a->m1 * a->m2 * a->m3;
   const size_t fsz = sizeof(float) * n3d;

@@ -69,6 +69,48 @@ def test_invalid_arguments_are_reported_not_aborted():
     assert b"empty" in L.brams_chem_last_error()
 
 
+@pytest.mark.parametrize("entry", ["brams_chem_rodas3_dyndt", "brams_chem_ros_dyndt"])
+def test_host_step_refuses_null_arrays_before_device_work(entry):
+    """A missing array of a host step is refused with -2: it must neither be
+    read nor leave the device computing on what an earlier call brought."""
+    from brams_amd.mechanism import load_mechanism
+    m, g, L = load_mechanism(), Grid(4, 4, 4), abi.lib()
+    n3d = g.m1 * g.m2 * g.m3
+    f32, f64 = np.zeros(m.nr_photo * n3d, np.float32), np.zeros(m.nr_photo * n3d, np.float64)
+    index = np.arange(1, m.nspecies + 1, dtype=np.int32)
+    fp = C.POINTER(C.c_float)
+
+    def args(split="SYMMETRIC", ndyn=1):
+        a = abi.ChemArgs()
+        a.m1, a.m2, a.m3, a.ia, a.iz, a.ja, a.jz = g.m1, g.m2, g.m3, g.ia, g.iz, g.ja, g.jz
+        a.dtlt, a.n_dyn_chem, a.split_method = 60.0, ndyn, abi.SPLIT[split]
+        a.nspecies, a.nr, a.nr_photo = m.nspecies, m.nr, m.nr_photo
+        a.n_transported, a.n_not_transported = m.nspecies, 1
+        a.nob, a.maxblock_size = 1, 64
+        for name, kind in abi.ChemArgs._fields_:
+            if kind is fp:
+                setattr(a, name, f32.ctypes.data_as(kind))
+            elif kind is C.POINTER(C.c_double):
+                setattr(a, name, f64.ctypes.data_as(kind))
+            elif kind is C.POINTER(C.c_int32):
+                setattr(a, name, index.ctypes.data_as(kind))
+        a.tables = [(fp * m.nspecies)(*[f32.ctypes.data_as(fp)] * m.nspecies) for _ in range(3)]
+        a.sc_p, a.sc_t, a.sc_t_dyn = (C.cast(t, C.POINTER(fp)) for t in a.tables)
+        return a
+
+    for name in ("pp", "pi0", "theta", "rv", "jphoto", "weight", "transp_chem_index", "no_transp_chem_index", "sc_p",
+                 "block_end", "last_accepted_dt", "atol", "rtol"):
+        a = args()
+        setattr(a, name, None)
+        assert getattr(L, entry)(C.byref(a)) == -2, name
+        assert b"null argument" in L.brams_chem_last_error(), name
+    for table, split, ndyn in ((0, "SYMMETRIC", 1), (1, "PARALLEL", 1), (2, "PARALLEL", 2)):
+        a = args(split, ndyn)
+        a.tables[table][m.nspecies - 1] = None
+        assert getattr(L, entry)(C.byref(a)) == -2, table
+        assert b"species %d" % m.nspecies in L.brams_chem_last_error()
+
+
 def test_surrogate_step_rejects_parallel_split():
     """brams_sur_step writes accepted cells straight into sc_p (the
     SYMMETRIC/SEQUENTIAL write-back, rodas3:774-798), so a PARALLEL call is
