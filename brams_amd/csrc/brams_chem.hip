@@ -1458,11 +1458,13 @@ int brams_chem_tuv_jphoto_device(const brams_tuv_map_args* a) {
   HIP_TRY(hipEventRecord(g.ev0, st));
   brams::TuvTiles q{};
   q.lev = (unsigned)((a->m1 + brams::kTuvLevels - 1) / brams::kTuvLevels);
-  q.col = (unsigned)((ni + brams::kTuvCols - 1) / brams::kTuvCols);
-  q.tiles = (unsigned)(q.lev * q.col * nj);
+  q.tiles = (unsigned)(q.lev * ((ni * nj + brams::kTuvCols - 1) / brams::kTuvCols));
   q.chunk = (q.tiles + brams::kXcds - 1) / brams::kXcds;
-  const unsigned frame = (unsigned)((n3d - npts + 255) / 256);
-  hipLaunchKernelGGL(brams::tuv_map, dim3(q.chunk * brams::kXcds + frame), dim3(256), 0, st, p, q);
+  // a dispatch counts its work-items in 32 bits a dimension: rows of 2^23
+  // workgroups, the last one padded (a workgroup behind the frame does nothing)
+  constexpr unsigned kRow = 1u << 23;
+  const unsigned n = q.chunk * brams::kXcds + (unsigned)((n3d - npts + 255) / 256);
+  hipLaunchKernelGGL(brams::tuv_map, dim3(std::min(n, kRow), (n + kRow - 1) / kRow), dim3(256), 0, st, p, q);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(g.ev1, st));
   HIP_TRY(hipStreamSynchronize(st));

@@ -34,23 +34,24 @@ struct TuvMapParams {
 // every XCD works through one contiguous run of tiles, and neighbouring tiles,
 // which share 128-byte lines of both arrays, go through one L2.
 constexpr int kXcds = 8;
-__device__ __forceinline__ unsigned xcd_tile(unsigned chunk) {
-  return (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds;
-}
+__device__ __forceinline__ unsigned xcd_tile(unsigned w, unsigned chunk) { return (w % kXcds) * chunk + w / kXcds; }
 
 // valJLoc has the column fastest, jphoto the rate and then the level, so the
-// mapping is a transpose.  A tile is kTuvCols neighbouring columns times
-// kTuvLevels levels, one thread a point: a wave reads two runs of 256 bytes of
-// valJLoc, the relations apply in registers, and the rates go through LDS to
+// mapping is a transpose.  A tile is kTuvCols consecutive interior columns (i,
+// then j, as valJLoc has them without gaps, so that a narrow interior fills
+// its tiles too) times kTuvLevels levels, one thread a point: a wave reads two
+// runs of 256 bytes of valJLoc, the relations apply in registers, and the rates go through LDS to
 // be written in runs of kTuvLevels * MECH_NPHOT values (1088 bytes).  The odd
 // row length keeps the LDS columns on different banks.  HBM bound: 200x200x40
-// (453 MB) takes 117 us with its launch, 3.9 TB/s where a large copy reaches
+// (453 MB) takes 116 us with its launch, 3.9 TB/s where a large copy reaches
 // 4.65; with a thread writing its 136 bytes directly, which touched 64 lines
-// with every load and store, 162 us.
+// with every load and store, 170 us.  40000 columns as 2x20000 (whose frame
+// has as many) take 209 us, 249 with a thread a point and 443 with tiles that
+// end with the row of i.
 constexpr int kTuvCols = 32, kTuvLevels = 8, kTuvRow = kTuvLevels * MECH_NPHOT + (MECH_NPHOT * kTuvLevels % 2 == 0);
 
 struct TuvTiles {
-  unsigned lev, col, tiles, chunk;     // tiles along the levels and the columns of one j, in all, per XCD
+  unsigned lev, tiles, chunk;          // tiles along the levels, in all, per XCD
 };
 
 __device__ __forceinline__ void tuv_relations_at(double* jp) {
@@ -67,9 +68,11 @@ __device__ __forceinline__ void tuv_relations_at(double* jp) {
 // point: the relations alone, the entries they do not set unchanged.
 __global__ __launch_bounds__(256) void tuv_map(TuvMapParams p, TuvTiles q) {
   __shared__ double s[kTuvCols * kTuvRow];
+  __shared__ long long at[kTuvCols];                 // a column's first value in the tile's levels
   const int ni = p.iz - p.ia + 1, nj = p.jz - p.ja + 1;
-  if (blockIdx.x >= kXcds * q.chunk) {
-    const long long t = (long long)(blockIdx.x - kXcds * q.chunk) * 256 + threadIdx.x;
+  const unsigned w = blockIdx.y * gridDim.x + blockIdx.x;
+  if (w >= kXcds * q.chunk) {
+    const long long t = (long long)(w - kXcds * q.chunk) * 256 + threadIdx.x;
     long long c = t / p.m1;                          // column of the frame, j rows from the bottom
     const long long below = (long long)(p.ja - 1) * p.m2, side = p.m2 - ni;
     if (c >= (long long)p.m2 * p.m3 - (long long)ni * nj) return;
@@ -85,34 +88,34 @@ __global__ __launch_bounds__(256) void tuv_map(TuvMapParams p, TuvTiles q) {
     tuv_relations_at(p.jphoto + (long long)MECH_NPHOT * (t % p.m1 + p.m1 * c));
     return;
   }
-  const unsigned tile = xcd_tile(q.chunk);
+  const unsigned tile = xcd_tile(w, q.chunk);
   if (tile >= q.tiles) return;
   const int L0 = (int)(tile % q.lev) * kTuvLevels;
-  const unsigned tc = tile / q.lev;
-  const int i0 = (int)(tc % q.col) * kTuvCols, jj = (int)(tc / q.col);
-  const int nl = min(kTuvLevels, p.m1 - L0), nc = min(kTuvCols, ni - i0);
-  const int c = threadIdx.x % kTuvCols, l = threadIdx.x / kTuvCols;
-  // first value of the tile's column 0
-  double* out = p.jphoto + (long long)MECH_NPHOT * (L0 + (long long)p.m1 * ((p.ia - 1 + i0) + (long long)p.m2 * (p.ja - 1 + jj)));
-  const long long column = (long long)MECH_NPHOT * p.m1;
-  if (c < nc && l < nl) {
-    const int mz = L0 + l == 0 ? 0 : L0 + l - 1;     // level 1 repeats level 2
+  const unsigned cols = (unsigned)ni * (unsigned)nj, c0 = tile / q.lev * kTuvCols;
+  const int nl = min(kTuvLevels, p.m1 - L0);
+  const unsigned nc = min((unsigned)kTuvCols, cols - c0);
+  const unsigned c = threadIdx.x % kTuvCols, l = threadIdx.x / kTuvCols;
+  if (c < nc && (int)l < nl) {
+    const unsigned jj = (c0 + c) / (unsigned)ni, ii = c0 + c - jj * (unsigned)ni;
+    const long long first =
+        MECH_NPHOT * (L0 + (long long)p.m1 * ((p.ia - 1 + (int)ii) + (long long)p.m2 * (p.ja - 1 + (int)jj)));
+    if (l == 0) at[c] = first;
+    const int mz = L0 + l == 0 ? 0 : L0 + (int)l - 1;   // level 1 repeats level 2
     double v[MECH_NPHOT];
 #pragma unroll
     for (int n = 0; n < MECH_NPHOT; ++n) {
       const int k = p.src[n];
-      v[n] = k >= 0 ? p.valj[i0 + c + (long long)ni * (jj + (long long)nj * (k + (long long)p.kj * mz))]
-                    : out[c * column + l * MECH_NPHOT + n];
+      v[n] = k >= 0 ? p.valj[c0 + c + (long long)cols * (k + (long long)p.kj * mz)] : p.jphoto[first + l * MECH_NPHOT + n];
     }
     mech_j_relations(v);
 #pragma unroll
     for (int n = 0; n < MECH_NPHOT; ++n) s[c * kTuvRow + l * MECH_NPHOT + n] = v[n];
   }
   __syncthreads();
-  const unsigned run = (unsigned)nl * MECH_NPHOT, all = run * (unsigned)nc;
+  const unsigned run = (unsigned)nl * MECH_NPHOT, all = run * nc;
   for (unsigned e = threadIdx.x; e < all; e += 256) {
     const unsigned ec = e / run, er = e - ec * run;
-    out[ec * column + er] = s[ec * kTuvRow + er];
+    p.jphoto[at[ec] + er] = s[ec * kTuvRow + er];
   }
 }
 

@@ -54,10 +54,12 @@ def test_tuv_mapping_16x16x10_bit_identical(kind):
     assert np.array_equal(gpu, ref)
 
 
-@pytest.mark.parametrize("nx,ny,nz,lo,hi", [(1, 1, 1, 0, 0), (33, 3, 7, 0, 0), (31, 2, 6, 2, 1), (64, 5, 14, 1, 3)])
+@pytest.mark.parametrize("nx,ny,nz,lo,hi", [(1, 1, 1, 0, 0), (33, 3, 7, 0, 0), (31, 2, 6, 2, 1), (64, 5, 14, 1, 3),
+                                             (1, 65, 3, 0, 0), (2, 37, 9, 1, 0), (5, 13, 16, 0, 2)])
 def test_tuv_mapping_ragged_tiles_bit_identical(nx, ny, nz, lo, hi):
-    """Columns and levels that leave part of a tile empty, interiors that
-    start and end off the grid's second column, and rates that no reaction
+    """Columns and levels that leave part of a tile empty, tiles that hold
+    several rows of a narrow interior, interiors that start and end off the
+    grid's second column, and rates that no reaction
     writes (they keep their values)."""
     print("case tuv mapping %dx%dx%d +%d +%d" % (nx, ny, nz, lo, hi), flush=True)
     grid = Grid(nx, ny, nz)
@@ -73,6 +75,31 @@ def test_tuv_mapping_ragged_tiles_bit_identical(nx, ny, nz, lo, hi):
     rc, gpu, _ = _run(grid, valj, xref, before)
     assert rc == 0
     assert np.array_equal(gpu, O.tuv_jphoto(grid, valj, xref, before))
+
+
+def test_tuv_mapping_of_a_narrow_interior_keeps_its_rate():
+    """40000 columns as 2x20000 and as 200x200: the narrow grid has a frame as
+    large as its interior, so it takes about twice the time (1.8 measured); with
+    30 of 32 threads of a tile idle it took 3.8 times."""
+    import torch
+    from brams_amd import abi
+    from brams_amd.chem import tuv_jphoto_device
+    ms = []
+    for nx, ny in ((200, 200), (2, 20000)):
+        print("case tuv mapping %dx%dx40, timed" % (nx, ny), flush=True)
+        grid, kj, kz = Grid(nx, ny, 40), 20, 42
+        valj = torch.rand((kz, kj, ny, nx), device="cuda", dtype=torch.float64)
+        jphoto = torch.rand((grid.m3, grid.m2, grid.m1, NP), device="cuda", dtype=torch.float64)
+        xref = np.zeros(kj, np.int32)
+        xref[:NP] = np.arange(1, NP + 1)
+        times = []
+        for _ in range(10):
+            assert tuv_jphoto_device(grid, valj, kj, kz, xref, jphoto) == 0
+            times.append(abi.stats().kernel_ms)
+        ms.append(min(times))
+        del valj, jphoto
+    print("  %.3f and %.3f ms" % tuple(ms), flush=True)
+    assert ms[1] < 2.8 * ms[0]
 
 
 def test_tuv_mapping_200x200x40_bit_identical():
