@@ -116,10 +116,12 @@ MLP_BYTES_PER_CELL = 1825
 
 
 def block_kernel(solver="rodas3"):
-    """Name of the kernel that runs the blocks of at most 64 cells."""
+    """Name of the kernel that ran the blocks of at most 64 cells in the last step."""
+    from brams_amd import abi
     from brams_amd.mechanism import default_name
     if default_name() == "racm_tuv":                    # one lane to a cell
-        return ("ros2_blocks<64,%d>" if solver == "ros2" else "rodas3_blocks<64,false,%d>") % 4
+        waves = {3: 1, 5: 4}[abi.stats().kernel_form]
+        return ("ros2_blocks<64,%d>" if solver == "ros2" else "rodas3_blocks<64,false,%d>") % waves
     return "coop_blocks<%d,false,false>" % (1 if solver == "ros2" else 0)
 
 

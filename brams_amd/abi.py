@@ -187,7 +187,7 @@ def block_thresholds(nob):
 
 
 def set_form(form):
-    """Kernel form of the 64-cell blocks (-1: none forced); see brams_chem_set_form."""
+    """Kernel form of the 64-cell blocks (-1: the library's choice); see brams_chem_set_form."""
     check(lib().brams_chem_set_form(form), "brams_chem_set_form")
 
 

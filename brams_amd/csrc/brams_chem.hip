@@ -29,6 +29,10 @@
 
 namespace {
 
+using brams::kFirstForm;
+using brams::kForms;
+using brams::form_built;
+
 thread_local std::string g_err = "";
 
 int fail(int code, const char* fmt, ...) {
@@ -89,16 +93,6 @@ struct HostBuf {
   }
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
-
-// Kernel forms of the 64-cell blocks, by the numbers that callers know
-// (brams_chem_set_form).  0..2 were layouts that never ran; 3..5 were register
-// budgets of a one-lane-per-cell kernel.  The cooperative block kernel has one
-// form, so all of 3..5 run it and there is nothing to choose.
-constexpr int kFirstForm = 3;
-constexpr int kForms = 6;
-constexpr bool form_built(int f) {
-  return f >= kFirstForm && f < kForms && (!brams::kLeanBuild || f != kFirstForm + 1);
-}
 
 // Device state of one grid, created on the first call for that grid and
 // kept until brams_chem_finalize (the reference allocates its block index
@@ -371,7 +365,7 @@ int launch_step(brams::StepParams p, hipStream_t st) {
   int nbig = 0;
   while (nbig < nob && sz[nbig] > 64) ++nbig;
   const int first64 = nbig > 1 ? nbig : 1;
-  const int form = g.force_form >= 0 ? g.force_form : kFirstForm;
+  const int form = brams::block_form((unsigned)(nob - first64), g.force_form);
   int rc = ensure_halves(nbig, p);
   if (rc) return rc;
   // the 64-cell blocks run longest first once a call on this grid has
@@ -389,7 +383,7 @@ int launch_step(brams::StepParams p, hipStream_t st) {
   g.main_cells = 0;
   if (nob > first64) {
     p.block_order = order;
-    HIP_TRY(brams::launch_rodas3((unsigned)(nob - first64), p, first64, st));
+    HIP_TRY(brams::launch_rodas3((unsigned)(nob - first64), p, first64, st, form));
     for (int b = first64; b < nob; ++b) g.main_cells += sz[b];
   }
   HIP_TRY(hipEventRecord(g.ev1, st));
@@ -435,7 +429,7 @@ int launch_ros2_step(brams::StepParams p, hipStream_t st) {
   // ROS2 never had a form 4
   if (g.force_form == kFirstForm + 1)
     return fail(-6, "ROS2 has no kernel form %d", g.force_form);
-  const int form = g.force_form >= 0 ? g.force_form : kFirstForm;
+  const int form = brams::block_form((unsigned)(nob - nbig), g.force_form);
   int rc = ensure_halves(nbig, p);
   if (rc) return rc;
   const int* order = nullptr;
@@ -451,7 +445,7 @@ int launch_ros2_step(brams::StepParams p, hipStream_t st) {
   if (nob > nbig) {
     brams::StepParams pm = p;
     pm.block_order = order;
-    HIP_TRY(brams::launch_ros2((unsigned)(nob - nbig), pm, nbig, st));
+    HIP_TRY(brams::launch_ros2((unsigned)(nob - nbig), pm, nbig, st, form));
     for (int b = nbig; b < nob; ++b) g.main_cells += gs.sizes[b];
   }
   HIP_TRY(hipEventRecord(g.ev1, st));

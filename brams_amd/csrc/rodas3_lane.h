@@ -24,8 +24,7 @@
 
 namespace brams {
 
-constexpr int kLaneManyWaves = 4;        // WPS of large launches
-constexpr unsigned kLaneManyBlocks = 4096;    // from this many blocks on
+constexpr int kLaneManyWaves = 4;        // WPS of large launches (form 5, rodas3_launch.h)
 
 template <int WG>
 __device__ __forceinline__ void block_reduce(double& errmax, int& rej, int& fail,

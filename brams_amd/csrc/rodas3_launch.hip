@@ -10,13 +10,13 @@
 
 namespace brams {
 
-hipError_t launch_rodas3(unsigned nblocks, const StepParams& p, int block0, hipStream_t st) {
+hipError_t launch_rodas3(unsigned nblocks, const StepParams& p, int block0, hipStream_t st, [[maybe_unused]] int form) {
   if (nblocks == 0) return hipSuccess;
 #ifdef BRAMS_MECH_COOP
   return coop_launch<kRodas3, false, false>(nblocks, p, block0, st);
 #else
   if (p.cell_list) return hipErrorInvalidValue;
-  if (nblocks >= kLaneManyBlocks)
+  if (block_form(nblocks, form) == kFormFourWaves)
     hipLaunchKernelGGL((rodas3_blocks<64, false, kLaneManyWaves>), dim3(nblocks), dim3(64), 0, st, p, block0);
   else
     hipLaunchKernelGGL((rodas3_blocks<64, false, 1>), dim3(nblocks), dim3(64), 0, st, p, block0);

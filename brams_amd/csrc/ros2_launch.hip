@@ -10,12 +10,12 @@
 
 namespace brams {
 
-hipError_t launch_ros2(unsigned nblocks, const StepParams& p, int block0, hipStream_t st) {
+hipError_t launch_ros2(unsigned nblocks, const StepParams& p, int block0, hipStream_t st, [[maybe_unused]] int form) {
   if (nblocks == 0) return hipSuccess;
 #ifdef BRAMS_MECH_COOP
   return coop_launch<kRos2, false, false>(nblocks, p, block0, st);
 #else
-  if (nblocks >= kLaneManyBlocks)
+  if (block_form(nblocks, form) == kFormFourWaves)
     hipLaunchKernelGGL((ros2_blocks<64, kLaneManyWaves>), dim3(nblocks), dim3(64), 0, st, p, block0);
   else
     hipLaunchKernelGGL((ros2_blocks<64, 1>), dim3(nblocks), dim3(64), 0, st, p, block0);

@@ -312,11 +312,13 @@ int brams_chem_block_status(int32_t *attempts, int32_t *substeps, int32_t *faile
 int brams_chem_block_thresholds(int32_t *counts, int32_t max_nob);
 
 /*
- * Kernel form of the 64-cell blocks (no reference counterpart): -1 (default)
- * or one of 3, 4 and 5, kept for callers that force one.  All run the same
- * kernel with the same results.  0..2 are refused (-6); the ROS2 step has no
- * form 4 (its calls fail with -6 while it is forced), nor has a lean library
- * (libbrams_chem_<mech>.so), which refuses it here (-6).
+ * Kernel form of the 64-cell blocks in the one-grid steps (no reference
+ * counterpart): -1 (default) or one of 3, 4 and 5.  In the libraries of
+ * RELACS_TUV, RELACS_MX and CB07_TUV these are one kernel.  RACM_TUV's has two
+ * register budgets with bit-identical results: 3 allows one wave per SIMD, 5
+ * four; -1 takes 5 from 4096 blocks on.  0..2 are refused (-6); the ROS2 step
+ * has no form 4 (its calls fail with -6 while it is forced), nor has a lean
+ * library (libbrams_chem_<mech>.so), which refuses it here (-6).
  */
 int brams_chem_set_form(int32_t form);
 /* The current grid's form, and the time (ms) of the 64-cell blocks in the

@@ -209,6 +209,39 @@ def gpu():
         say("GPU split write-back %s N_DYN_CHEM=%d through the host entry: worst %.2g (oracle's one-ulp "
             "sensitivity %.2g)" % (method, ndyn, worst, sens))
     fortran_drop_ins()
+    if MECH.name == "RACM_TUV":
+        lane_forms()
+
+
+def lane_forms():
+    """RACM_TUV's kernel forms 3 and 5 (one and four waves per SIMD): forced,
+    each reports itself and gives the other's results bit for bit; by default
+    the number of 64-cell blocks chooses, 5 from 4096 on; forced on 4160 blocks
+    of the ROS2 step, 3 takes longer than 5 (measured 523 against 393 ms), so
+    forcing reaches the kernel."""
+    import torch
+    from brams_amd import abi
+    from brams_amd.chem import DeviceStep
+
+    def step(wl, tol, solver, form):
+        abi.set_form(form)
+        ds = DeviceStep(wl, *tolerances(tol), solver=solver)
+        rc = ds.step()
+        return rc, ds.sc_p, ds.last_dt, abi.stats()
+
+    small = make_workload(Grid(24, 24, 10), seed=2, sza="split")
+    large = make_workload(Grid(64, 130, 32), seed=3, sza="split")
+    try:
+        for solver in ("rodas3", "ros2"):
+            (rc, sc, dt, st), (rc5, sc5, dt5, st5), (_, _, _, st0) = (step(small, "baseline", solver, f) for f in (3, 5, -1))
+            assert rc == rc5 and (st.kernel_form, st5.kernel_form, st0.kernel_form) == (3, 5, 3), solver
+            assert torch.equal(sc, sc5) and torch.equal(dt, dt5), solver
+            assert step(large, "reference", solver, -1)[3].kernel_form == 5, solver
+        ms = [min(step(large, "reference", "ros2", f)[3].main_ms for _ in range(2)) for f in (3, 5)]
+        assert ms[0] > 1.15 * ms[1], ms
+    finally:
+        abi.set_form(-1)
+    say("GPU forms 3 and 5: bit-identical on 24x24x10, ROS2 on 64x130x32 %.0f and %.0f ms" % tuple(ms))
 
 
 def fortran_drop_ins():
