@@ -192,8 +192,8 @@ def set_form(form):
 
 
 def tuning():
-    """(kernel form of the current grid, ms of its first call's 64-cell blocks
-    per built form: they are one kernel)."""
+    """(kernel form of the current grid's last RODAS3 step, ms of the 64-cell
+    blocks in its first RODAS3 step per form); see brams_chem_get_tuning."""
     import numpy as np
     f = np.zeros(1, np.int32)
     ms = np.zeros(8, np.float32)

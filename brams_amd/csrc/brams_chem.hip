@@ -121,7 +121,8 @@ struct GridState {
   DevBuf cell_dt;
   std::vector<int> h_att, h_sub, h_fail, h_thresh;
   std::vector<float> h_forced;
-  float tune_ms[kForms] = {};    // 64-cell blocks of the grid's first RODAS3 call
+  int form = -1;                 // of the last one-grid RODAS3 step
+  float tune_ms[kForms] = {};    // 64-cell blocks of the first such step with each form
   bool same(int a1, int a2, int a3, int b1, int b2, int b3, int b4) const {
     return m1 == a1 && m2 == a2 && m3 == a3 && ia == b1 && iz == b2 && ja == b3 && jz == b4;
   }
@@ -495,10 +496,20 @@ int collect_stats(hipStream_t st) {
   s.main_ms = ms;
   s.main_cells = g.main_cells;
   s.kernel_form = g.last_form;
-  for (int f = kFirstForm; f < kForms; ++f)
-    if (form_built(f) && gs.tune_ms[f] == 0.f) gs.tune_ms[f] = ms;
   g.stats = s;
   return (int)s.failed_blocks;
+}
+
+// collect_stats() of a one-grid RODAS3 step, whose form and time
+// brams_chem_get_tuning reports
+int collect_rodas3(hipStream_t st) {
+  const int rc = collect_stats(st);
+  if (rc < 0 || g.last_form < 0) return rc;
+  GridState& gs = *g.cur;
+  gs.form = g.last_form;
+  for (int f = kFirstForm; f < kForms; ++f)
+    if (form_built(f) && (brams::kOneForm || f == g.last_form) && gs.tune_ms[f] == 0.f) gs.tune_ms[f] = g.stats.main_ms;
+  return rc;
 }
 
 // grid, photolysis method and time step: the checks every solver shares
@@ -763,7 +774,7 @@ int brams_chem_rodas3_dyndt_device(const brams_chem_dev_args* a) {
   if (rc) return rc;
   hipStream_t st = (hipStream_t)a->stream;
   if ((rc = launch_step(p, st))) return rc;
-  return collect_stats(st);
+  return collect_rodas3(st);
 }
 
 // The same step with no allocation: the bookkeeping sits in `scratch`, the
@@ -1316,7 +1327,7 @@ int host_step(const brams_chem_args* a, int solver) {
   if ((rc = solver == brams::kRos2 ? launch_ros2_step(p, st) : launch_step(p, st))) return rc;
   // results back into the caller's arrays
   if ((rc = h.fetch(st))) return rc;
-  if ((rc = collect_stats(st)) >= 0) h.unpack();
+  if ((rc = solver == brams::kRos2 ? collect_stats(st) : collect_rodas3(st)) >= 0) h.unpack();
   return rc;
 }
 
@@ -1540,7 +1551,7 @@ int brams_chem_set_form(int32_t form) {
 
 int brams_chem_get_tuning(int32_t* form, float* ms, int32_t n) {
   if (!g.cur) return fail(-2, "no chemistry step has run");
-  if (form) *form = kFirstForm;
+  if (form) *form = g.cur->form;
   for (int f = 0; f < n && f < kForms && ms; ++f) ms[f] = g.cur->tune_ms[f];
   return kForms;
 }

@@ -38,7 +38,10 @@ constexpr int kFirstForm = 3;
 constexpr int kFormFourWaves = 5;
 constexpr int kForms = 6;
 constexpr bool form_built(int f) { return f >= kFirstForm && f < kForms && (!kLeanBuild || f != kFirstForm + 1); }
-#ifndef BRAMS_MECH_COOP
+#ifdef BRAMS_MECH_COOP
+constexpr bool kOneForm = true;
+#else
+constexpr bool kOneForm = false;
 // From this many blocks on, the one-lane-per-cell kernel takes the budget of
 // four waves per SIMD: up to 1024 blocks run at once with one wave per SIMD
 // and all of them sooner, then the waves that hide each other's spill traffic

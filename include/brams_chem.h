@@ -321,9 +321,11 @@ int brams_chem_block_thresholds(int32_t *counts, int32_t max_nob);
  * library (libbrams_chem_<mech>.so), which refuses it here (-6).
  */
 int brams_chem_set_form(int32_t form);
-/* The current grid's form, and the time (ms) of the 64-cell blocks in the
- * grid's first call, for each form that the library has (0: none), into
- * ms[0..n); returns the number of forms. */
+/* The form of the current grid's last RODAS3 step (-1: none), and the time (ms)
+ * of the 64-cell blocks in its first RODAS3 step with each form (0: none; where
+ * the forms are one kernel, that of the first step under each that the library
+ * has) into ms[0..n); steps of several grids do not count.  Returns the number
+ * of forms. */
 int brams_chem_get_tuning(int32_t *form, float *ms, int32_t n);
 
 /* Text of the last error (thread-local, never NULL). */

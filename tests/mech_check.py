@@ -237,6 +237,8 @@ def lane_forms():
             assert rc == rc5 and (st.kernel_form, st5.kernel_form, st0.kernel_form) == (3, 5, 3), solver
             assert torch.equal(sc, sc5) and torch.equal(dt, dt5), solver
             assert step(large, "reference", solver, -1)[3].kernel_form == 5, solver
+            form, ms = abi.tuning()                       # RODAS3 steps alone, the one form that ran
+            assert form == 5 and list(np.nonzero(ms)[0]) == [5], (form, ms)
         ms = [min(step(large, "reference", "ros2", f)[3].main_ms for _ in range(2)) for f in (3, 5)]
         assert ms[0] > 1.15 * ms[1], ms
     finally:
