@@ -165,12 +165,11 @@ def free(expr):
 
 
 class Plan:
-    """Which wave owns which row, and where the rate constants live."""
+    """Which wave owns which row, and the LDS slots that hold a value throughout."""
 
-    def __init__(self, m, waves, dense, row_wave, rk_regs, rk_lit=None):
+    def __init__(self, m, waves, dense, row_wave, rk_lit=None):
         self.m, self.waves, self.dense, self.t0 = m, waves, dense, m.ns - dense
         self.row_wave, self.dw = row_wave, waves - 1         # by pivot position; the dense wave
-        self.rk_regs = rk_regs
         self.rk_lit = rk_lit or {}                           # constants that depend on nothing
         self.own = [[] for _ in range(waves)]                # species of each wave
         for I, w in enumerate(row_wave):
@@ -184,27 +183,12 @@ class Plan:
         for w in range(waves):
             for r in self.need[w]:
                 users.setdefault(r, []).append(w)
-        self.rk_users = users
-        # the constants with the fewest users stay in those waves' registers,
-        # up to rk_regs of each wave; the others sit in LDS
-        held = [0] * waves
-        self.rk_reg = [dict() for _ in range(waves)]
-        self.rk_lds = []
-        cap = [rk_regs if w != self.dw else min(rk_regs, 12) for w in range(waves)]
-        for r in sorted(users, key=lambda r: (len(users[r]), r)):
-            if r in self.rk_lit:
-                continue
-            if all(held[w] < cap[w] for w in users[r]):
-                for w in users[r]:
-                    self.rk_reg[w][r] = held[w]
-                    held[w] += 1
-            else:
-                self.rk_lds.append(r)
-        # persistent slots: the concentrations, then the LDS rate constants
+        # the rate constants, those with the fewest users first
+        self.rk_lds = [r for r in sorted(users, key=lambda r: (len(users[r]), r)) if r not in self.rk_lit]
+        # persistent slots: the concentrations, then the rate constants
         self.yslot = {s: s for s in range(m.ns)}
         self.rkslot = {r: len(self.yslot) + k for k, r in enumerate(self.rk_lds)}
         self.nfix = len(self.yslot) + len(self.rkslot)
-        self.nrk = [max(1, len(d)) for d in self.rk_reg]
         self.mask_own = [dict() for _ in range(waves)]       # mask words of each wave's rows
 
 
@@ -219,11 +203,8 @@ class Builder:
         for r, v in self.rkl.items():
             v.slot = plan.rkslot[r]
 
-    def rk(self, w, r):
-        if r in self.p.rk_lit:
-            return free(self.p.rk_lit[r])
-        k = self.p.rk_reg[w].get(r)
-        return free("rk[%d]" % k) if k is not None else self.rkl[r]
+    def rk(self, r):
+        return free(self.p.rk_lit[r]) if r in self.p.rk_lit else self.rkl[r]
 
     def add_rate(self, w, acc, rows, r, t, last):
         """Adds the rate t * last of reaction r to the sums of `rows`."""
@@ -256,7 +237,7 @@ class Builder:
             for r in p.need[w]:
                 rows = [s for s in p.own[w] if (s, r) in m.coef]
                 rs = m.react[r]
-                t = self.rk(w, r)
+                t = self.rk(r)
                 for s in rs[:-1]:
                     t = f.op(w, "{0} * {1}", [t, yv[s]])
                 self.add_rate(w, acc, rows, r, t, yv[rs[-1]])
@@ -276,10 +257,10 @@ class Builder:
                 """d(rate r)/d(its reactant in `slot`)"""
                 rs = m.react[r]
                 if len(rs) == 1:
-                    return self.rk(w, r)
+                    return self.rk(r)
                 o = rs[1 - slot]
                 if (r, o) not in prods:
-                    prods[(r, o)] = f.op(w, "{0} * {1}", [self.rk(w, r), self.yc[o]])
+                    prods[(r, o)] = f.op(w, "{0} * {1}", [self.rk(r), self.yc[o]])
                 return prods[(r, o)]
 
             for r in p.need[w]:
@@ -698,12 +679,6 @@ def emit(m, plan, reactions, rate_line, name, mech_name):
         lay = Layout(b.f, plan.nfix, W)
         secs[solver] = lay
         slots = max(slots, lay.slots)
-    # rate constants on their way from the wave that evaluates them to the
-    # registers of those that use them: the exchange slots, free at that time
-    reg_rk = sorted({r for d in plan.rk_reg for r in d})
-    used = [r for r in sorted(plan.rk_users) if r not in plan.rk_lit]
-    tmp = {r: plan.nfix + k for k, r in enumerate(reg_rk)}
-    slots = max(slots, plan.nfix + len(reg_rk))
     eslot = slots
     slots += W                       # error partials
     vslot = slots
@@ -716,8 +691,9 @@ def emit(m, plan, reactions, rate_line, name, mech_name):
     w_("// Generated by brams_amd/codegen/gen_coop.py from brams_amd/mechanism/%s.json." % name)
     w_("// One block's attempt spread over %d waves: RODAS3 in %d phases, ROS2 in %d;" % (
         W, secs["rodas3"].P, secs["ros2"].P))
-    w_("// the last %d pivots on wave %d; %d of %d rate constants in LDS." % (
-        plan.dense, plan.dw, len(plan.rk_lds), len(used)))
+    w_("// the last %d pivots on wave %d; %d rate constants in LDS.  Modelled clocks of an" % (
+        plan.dense, plan.dw, len(plan.rk_lds)))
+    w_("// attempt, barriers included: %d and %d." % (secs["rodas3"].stats()[0], secs["ros2"].stats()[0]))
     w_("#pragma once")
     w_("#define MECH_COOP_WAVES %d" % W)
     w_("#define MECH_COOP_SLOTS %d" % slots)
@@ -726,13 +702,13 @@ def emit(m, plan, reactions, rate_line, name, mech_name):
     w_("#define MECH_COOP_VWORDS %d" % vwords)
     w_("#define MECH_COOP_MSLOT %d" % mslot)
     w_("")
-    shares = kinetic_shares(W, {r: law_cost(reactions[r]["rate"]) for r in used})
+    shares = kinetic_shares(W, {r: law_cost(reactions[r]["rate"]) for r in plan.rk_lds})
     nwords = (len(m.sidx) + 31) // 32
     for w in range(W):
         own = plan.own[w]
         n = max(1, len(own))
         w_("struct CoopWave%d {" % w)
-        w_("  static constexpr int kOwn = %d, kRk = %d;" % (len(own), plan.nrk[w]))
+        w_("  static constexpr int kOwn = %d;" % len(own))
         w_("  // species (0-based); a species' concentration lies in the slot of its number")
         w_("  static constexpr int own[%d] = {%s};" % (n, ", ".join(map(str, own)) or "0"))
         mo = [plan.mask_own[w].get(q, 0) for q in range(nwords)]
@@ -744,18 +720,11 @@ def emit(m, plan, reactions, rate_line, name, mech_name):
         w_("    const double lnT = log(T);")
         w_("    (void)M; (void)H2O; (void)lnT; (void)J;")
         for r in shares[w]:
-            sl = plan.rkslot.get(r, tmp.get(r))
-            w_("    S.put(%d, %s);" % (sl, rate_line(r)))
-        w_("  }")
-        w_("  static __device__ __forceinline__ void load_rk(const CoopLds& S, double* rk) {")
-        if not plan.rk_reg[w]:
-            w_("    rk[0] = 0.0;")
-        for r, k in sorted(plan.rk_reg[w].items(), key=lambda t: t[1]):
-            w_("    rk[%d] = S.get(%d);" % (k, tmp[r]))
+            w_("    S.put(%d, %s);" % (plan.rkslot[r], rate_line(r)))
         w_("  }")
         for solver in ("rodas3", "ros2"):
             w_("  template <bool DYN, bool COUNT>")
-            w_("  static __device__ __forceinline__ void %s(const CoopLds& S, const double* rk," % solver)
+            w_("  static __device__ __forceinline__ void %s(const CoopLds& S," % solver)
             w_("      double igdt, double dti, unsigned* mw, bool dyn, const double* atol, const double* rtol,")
             w_("      double* yn, double& e, unsigned* viol) {")
             L.extend("  " + x for x in secs[solver].emit(w))

@@ -452,7 +452,7 @@ def emit_coop(m, ns, nr, react, prod, jt, perm, F, sidx, rate_rhs):
     if place is None:                    # runs one lane to a cell (rodas3_lane.h)
         return
     rows = place["rows"] or gen_coop.default_rows(mech, place["waves"], place["dense"])
-    plan = gen_coop.Plan(mech, place["waves"], place["dense"], rows, place["rk_regs"],
+    plan = gen_coop.Plan(mech, place["waves"], place["dense"], rows,
                          gen_coop.literal_rates(m["reactions"]))
     write(MECH + "_coop.h", gen_coop.emit(mech, plan, m["reactions"], rate_rhs, MECH, m["name"]))
 

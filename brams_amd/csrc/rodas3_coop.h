@@ -155,7 +155,7 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
   int* mbits = reinterpret_cast<int*>(lds + MECH_COOP_MSLOT * 64);
   (void)vbits;
 
-  double y[WV::kOwn + 1], yn[WV::kOwn + 1], rk[WV::kRk];
+  double y[WV::kOwn + 1], yn[WV::kOwn + 1];
   double* half = nullptr;                                 // [half][buffer][species][64]
   int cur = 0;
   if (COUNT && halves > 1) half = p.half_y + (long long)slot * (4 * MECH_NS * 64) + lane;
@@ -188,8 +188,6 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
     WV::kinetic(q.temp, q.press, q.vapp, p.jphoto + (long long)MECH_NPHOT * q.o, S);
     publish(y);
     coop_barrier();
-    WV::load_rk(S, rk);
-    coop_barrier();                                       // the slots are free for the exchange from here
   };
 
   const float tnf = p.dtlt * (float)p.ndyn;
@@ -241,9 +239,9 @@ __device__ __forceinline__ void coop_run(const StepParams& p, int b, int slot, d
           for (int k = 0; k < MECH_COOP_VWORDS; ++k) vbits[k * 64] = 0;
       }
       if constexpr (SOLVER == kRos2)
-        WV::template ros2<DYN, COUNT>(S, rk, igdt, dti, mw, false, p.atol, p.rtol, yn, e, viol);
+        WV::template ros2<DYN, COUNT>(S, igdt, dti, mw, false, p.atol, p.rtol, yn, e, viol);
       else
-        WV::template rodas3<DYN, COUNT>(S, rk, igdt, dti, mw, DYN && h == 0, p.atol, p.rtol, yn, e, viol);
+        WV::template rodas3<DYN, COUNT>(S, igdt, dti, mw, DYN && h == 0, p.atol, p.rtol, yn, e, viol);
       if (COUNT) {
         for (int k = 0; k < MECH_COOP_VWORDS; ++k) atomicOr(&vbits[k * 64], (int)viol[k]);
         if (halves > 1) {
