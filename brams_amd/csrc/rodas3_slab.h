@@ -1,7 +1,10 @@
 // FP64 RODAS3 for 64-cell blocks with explicit placement of the per-cell
-// working set ("slab kernel").
+// working set ("slab layout").  No library builds it: its kernels, persistent
+// workgroups that popped blocks from a device counter, did not terminate on
+// gfx950.  The integration of a block is kept for tests/test_slab_host.py, which
+// runs it on the host against the oracle.
 //
-// The per-lane kernel of rodas3_kernel.h keeps a cell's whole working set
+// The per-lane kernel of rodas3_lane.h keeps a cell's whole working set
 // (LU 534, rate constants 128, stage vectors) as locals, about 1000 doubles,
 // which the compiler spills to scratch however the registers are budgeted.
 // Here each piece has a fixed home, chosen by its reuse:
@@ -22,20 +25,15 @@
 //              every attempt's factorisation), the rate constants, f(y0)
 //              and the stage-4 right-hand-side part.
 //
-// The workgroups are persistent: a grid of slots (one slab each) pops block
-// indices from a device counter, in the order given (longest first from the
-// previous call's attempts, see sched_kernels.h), until the queue is empty.
-// Every block's arithmetic is that of rodas3_blocks operation for operation
-// (the generated functions of relacs_tuv_slab.h are checked bit for bit
-// against those of relacs_tuv_gen.h), so the results are bit-identical and
-// independent of which slot integrates which block.
+// A block's arithmetic is that of rodas3_blocks operation for operation (the
+// generated functions of relacs_tuv_slab.h are checked bit for bit against those
+// of relacs_tuv_gen.h), so the results are bit-identical.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include "mechanism.h"
 #include BRAMS_MECH_SLAB
 #include "rodas3_kernel.h"
-#include "rodas3_slab_launch.h"
 
 // Passes a value through an SGPR by an empty asm, so that the compiler
 // cannot hoist what is computed from it out of the enclosing loop (host
@@ -389,38 +387,6 @@ __device__ __forceinline__ void integrate_slab(const StepParams& p, int b, Lanes
     if (p.blk_forced) p.blk_forced[b] = forced;
     if (p.blk_thresh) p.blk_thresh[b] = v;
   }
-}
-
-// Persistent slots popping 64-cell blocks (LIST: 64-entry runs of
-// p.cell_list) from q.counter until q.nitems are taken.
-template <int NLDS, bool LIST, bool DYN>
-__global__ __launch_bounds__(64, 1) void rodas3_slab(StepParams p, QueueParams q) {
-  __shared__ double s_y[MECH_NS * 64];
-  __shared__ double s_lu[(NLDS > 0 ? NLDS : 1) * 64];
-  const int c = threadIdx.x;
-  const long long slot = blockIdx.x;
-  const Lanes ys{s_y + c};
-  const int lane8 = c * 8;
-  const LuLanes<NLDS> lu{s_lu + c,
-                         BufLanes{slab_rsrc(q.lu + slot * kSlabLuRows * 64, kSlabLuRows * 512LL), lane8}};
-  const BufLanes jac{slab_rsrc(q.jac + slot * kSlabJacRows * 64, kSlabJacRows * 512LL), lane8};
-  const BufLanes rkx{slab_rsrc(q.rk + slot * kSlabRkRows * 64, kSlabRkRows * 512LL), lane8};
-  const BufLanes f0{slab_rsrc(q.vec + slot * kSlabVecRows * 64, MECH_NS * 512LL), lane8};
-  const BufLanes p4{slab_rsrc(q.vec + slot * kSlabVecRows * 64 + MECH_NS * 64, MECH_NS * 512LL), lane8};
-  for (;;) {
-    int item = 0;
-    if (c == 0) item = atomicAdd(q.counter, 1);
-    item = __shfl(item, 0, 64);
-    if (item >= q.nitems) break;
-    const int b = q.order ? q.order[item] : q.b0 + item;
-    integrate_slab<NLDS, LIST, DYN>(p, b, ys, lu, jac, rkx, f0, p4);
-  }
-}
-
-// Sets the queue counter to zero (a kernel, not a memset, so that the
-// sequence can be captured in a graph).
-__global__ void queue_reset(int* counter) {
-  if (threadIdx.x == 0) counter[0] = 0;
 }
 
 }  // namespace brams
