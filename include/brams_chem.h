@@ -110,7 +110,7 @@ typedef struct brams_chem_stats {
     int64_t cell_substeps;       /* sum over cells of their block's accepted sub-steps */
     int64_t cell_attempts;       /* sum over cells of their block's attempts */
     float block1_ms;             /* device time of the block-1 kernel (mask, serial prefix) */
-    float main_ms;               /* device time of the wave64 kernel over the 64-cell blocks */
+    float main_ms;               /* device time of the kernel over the 64-cell blocks */
     int64_t main_cells;          /* cells that kernel integrated */
     int64_t forced_blocks;       /* blocks that accepted a step with error > 1 at dt_min */
     float max_forced_err;        /* largest such error (rodas3:671-676 accepts it) */

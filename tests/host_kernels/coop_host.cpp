@@ -1,6 +1,6 @@
 // Host emulation of the cooperative block kernels (rodas3_coop.h), for CPU
-// tests: one thread for every lane of every wave, with as many lanes as the
-// block has cells (of each half), so no lane is idle.  Barriers are barriers
+// tests: one thread for every lane of every wave, 64 lanes for a block of two
+// halves and else two more than it has cells: the others shadow cell 1.  Barriers are barriers
 // of the threads, the cross-lane operations go through shared arrays.
 #include <condition_variable>
 #include <cstdint>
@@ -114,7 +114,7 @@ extern "C" void coop_step_host(int solver, int m1, int m2, int m3, float dtlt, i
   p.half_y = half.data();
   for (int b = 0; b < nblk; ++b) {
     const int n = block_start[b + 1] - block_start[b];
-    g_lanes = n > 64 ? 64 : n;
+    g_lanes = n + 2 < 64 ? n + 2 : 64;
     g_group.n = g_lanes * MECH_COOP_WAVES;
     std::vector<std::thread> th;
     for (int w = 0; w < MECH_COOP_WAVES; ++w) {

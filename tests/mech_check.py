@@ -22,7 +22,8 @@ does; tests/test_mechanisms.py and tests/test_gpu_mechanisms.py start it).
          library against the C-ABI, bit for bit.
   --gpu-scale  the RODAS3 step at full depth against the oracle on sampled
          blocks (tests/test_gpu_scale_parity.py's check): 50x50x40 at dt
-         30 s, whose first 32 blocks have 65 cells (128-lane workgroups), and
+         30 s, whose first 32 blocks have 65 cells (two halves in turn, or
+         128 lanes for RACM_TUV), and
          the 1.6M-cell 200x200x40 grid; and the ROS2 and QSSA steps on that
          grid.
 
@@ -323,7 +324,7 @@ def gpu_scale():
     # error norm moves RACM_TUV's controller output by about 1e-9
     from test_gpu_scale_parity import run_case
     st = run_case(Grid(50, 50, 40, dtlt=30.0), "split", "baseline", every=25, head=40, dt_rtol=1e-6)
-    say("GPU RODAS3 50x50x40 (dt 30 s, 65-cell blocks on 128 lanes): sampled blocks = oracle, %.1f ms"
+    say("GPU RODAS3 50x50x40 (dt 30 s, 65-cell blocks): sampled blocks = oracle, %.1f ms"
         % st.kernel_ms)
     # without the x50 NOx/VOC plume: on CB07_TUV and RACM_TUV it blows up
     # hundreds of blocks (forced errors past 1e30), and which of them end that

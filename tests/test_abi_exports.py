@@ -130,9 +130,8 @@ def test_surrogate_step_rejects_parallel_split():
 
 
 def test_slab_forms_are_refused_while_switched_off():
-    """The slab kernel forms (0..2) are switched off in this build: the
-    per-lane forms (3, 4, 5: 1, 2, 4 waves per SIMD) and autotune (-1) are
-    accepted, a slab form is refused with an error and no device work."""
+    """Forms 0..2 (layouts that never ran) are refused with an error and no
+    device work; 3, 4 and 5 and the library's own choice (-1) are accepted."""
     L = abi.lib()
     assert L.brams_chem_set_form(0) == -6
     assert b"switched off" in L.brams_chem_last_error()

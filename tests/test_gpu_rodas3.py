@@ -84,8 +84,8 @@ def test_longest_first_block_order_changes_no_result():
 def test_nested_grid_shapes_match_oracle(nx, nz, dt):
     """The nested grids of the three-grid workload (98x98 and 50x50 columns,
     dt 60 s and 30 s) at reduced depth: AllocIndex gives them 65-cell blocks
-    (16 and 24 of them), which run as 128-lane workgroups with a two-wave
-    step-size reduction; split SZA and a plume, atol 1e-12 ppb."""
+    (16 and 24 of them), which run as two halves that share the step
+    size; split SZA and a plume, atol 1e-12 ppb."""
     print("case nested nx=%d nz=%d dt=%g" % (nx, nz, dt), flush=True)
     grid = Grid(nx, nx, nz, dtlt=dt)
     wl = make_workload(grid, seed=21, sza="split", plume_sigma=8.0)

@@ -3,8 +3,8 @@ against the oracle's ROS2 through the C-ABI.
 
 Checked: FP32 outputs within rel 1e-6 / abs 1e-12 ppb, attempts and
 accepted sub-steps equal, last_accepted_dt within rel 1e-9; the host entry
-equal to the device entry bit for bit; the 65-cell blocks of the nested
-shapes on 128 lanes; and the 1.6M-cell grid on 201 sampled blocks (ROS2 has
+equal to the device entry bit for bit; the nested shapes, whose first
+blocks have 65 cells; and the 1.6M-cell grid on 201 sampled blocks (ROS2 has
 no value mask, so every block is independent of the others).
 """
 import numpy as np

@@ -126,7 +126,7 @@ def run_case(grid, sza, tol, every, head=0, seed=0, dt_rtol=1e-9, plume=True, re
     assert nfail == 0, worst
     np.testing.assert_allclose(gdt[ids], hs.last_dt[ids], rtol=dt_rtol)
     # the GPU counts threshold-rule failures in block 1 and the 65..127-cell
-    # blocks (where Sparse1.3 orders, and the 128-lane kernel); the oracle in all
+    # blocks (where Sparse1.3 orders, and the two-half form); the oracle in all
     sizes = np.asarray(wl["block_end"])
     counted = ids[(ids == 0) | (sizes[ids] > 64)]
     assert np.array_equal(gth[counted], oth[counted])
@@ -137,8 +137,7 @@ def run_case(grid, sza, tol, every, head=0, seed=0, dt_rtol=1e-9, plume=True, re
 @pytest.mark.parametrize("tol", ["baseline", "reference"])
 @pytest.mark.parametrize("sza", ["split", "split_night_first"])
 def test_200x200x40_matches_oracle(sza, tol):
-    """The plain 1.6M-cell step (25 000 blocks, the autotuned per-lane
-    form); 501 sampled blocks plus block 1."""
+    """The plain 1.6M-cell step (25 000 blocks); 501 sampled blocks plus block 1."""
     st = run_case(Grid(200, 200, 40, dtlt=120.0), sza, tol, every=50)
     assert st.blocks == 25000
 
@@ -149,6 +148,6 @@ def test_200x200x40_matches_oracle(sza, tol):
                                            (50, 30.0, "split_night_first", "reference")])
 def test_nested_grids_full_depth_match_oracle(nx, dt, sza, tol):
     """The nested grids of the three-grid workload at full depth (40
-    levels): their first 32 blocks have 65 cells (128-lane workgroups) and
+    levels): their first 32 blocks have 65 cells (two halves) and
     are all sampled; 98x98x40 has 6002 blocks, 50x50x40 1562."""
     run_case(Grid(nx, nx, 40, dtlt=dt), sza, tol, every=25, head=40)

@@ -2,9 +2,9 @@
 on the same inputs, through the C-ABI: FP32 species, last_accepted_dt and
 the failed-block count bit-identical.  Three calls in a row on shrinking
 grids, so each call reuses what the previous one left in the entry's fixed
-device array: 98x98x4 (600 blocks, the first 16 of 65 cells on 128 lanes),
+device array: 98x98x4 (600 blocks, the first 16 of 65 cells),
 16x16x10 (40 blocks of 64), 7x19x1 (two blocks of 67 and 66 cells, every
-block on 128 lanes)."""
+block in two halves)."""
 import ctypes as C
 
 import numpy as np
