@@ -103,15 +103,22 @@ def qssa_flop_model(itchim):
 QSSA_TRAFFIC_PER_CELL = 750 + 221
 # the same for tuv_map, bytes per interior grid point at kj 80, kz
 # 125 with 17 reactions mapped (profiles/kernel_stats_and_traffic.md)
-TUV_TRAFFIC_PER_POINT = 263
+TUV_TRAFFIC_PER_POINT = 262
 
 
 MLP_FLOP_PER_CELL = 3 * 2 * (68 * 256 + 3 * 256 * 256 + 256 * 47)
 BF16_PEAK_TFLOPS = 2500.0
-# HBM traffic of a block kernel per cell-attempt, measured with rocprofv3
-# --pmc FETCH_SIZE / WRITE_SIZE (scaled by the counters' reading of a 1 GiB
-# device copy), read + written; kernels without a measurement report null
-BYTES_PER_CELL_ATTEMPT = {}
+# HBM traffic of the block kernels, measured with rocprofv3 --pmc FETCH_SIZE /
+# WRITE_SIZE (scaled by the counters' reading of a 1 GiB device copy), read +
+# written (profiles/kernel_stats_and_traffic.md): a cooperative kernel's is the
+# same a cell whatever the attempts, a per-lane kernel's the same an attempt;
+# kernels without a measurement report null
+BYTES_PER_CELL = {("relacs_tuv", "coop_blocks<0,false,false>"): 522 + 780,
+                  ("relacs_tuv", "coop_blocks<1,false,false>"): 468 + 288}
+BYTES_PER_CELL_ATTEMPT = {("racm_tuv", "rodas3_blocks<64,false,4>"): 108800 + 31400,
+                          ("racm_tuv", "rodas3_blocks<64,false,1>"): 78400 + 19100,
+                          ("racm_tuv", "ros2_blocks<64,4>"): 69200 + 19000,
+                          ("racm_tuv", "ros2_blocks<64,1>"): 43500 + 12100}
 MLP_BYTES_PER_CELL = 1825
 
 
@@ -125,11 +132,13 @@ def block_kernel(solver="rodas3"):
     return "coop_blocks<%d,false,false>" % (1 if solver == "ros2" else 0)
 
 
-def block_traffic(kernel, cell_attempts):
-    """HBM bytes of a launch, where the kernel's bytes per attempt are measured."""
+def block_traffic(kernel, cells, cell_attempts):
+    """HBM bytes of a launch, where the kernel's are measured."""
     from brams_amd.mechanism import default_name
-    b = BYTES_PER_CELL_ATTEMPT.get((default_name(), kernel))
-    return None if b is None else b * cell_attempts
+    for table, n in ((BYTES_PER_CELL, cells), (BYTES_PER_CELL_ATTEMPT, cell_attempts)):
+        if (default_name(), kernel) in table:
+            return table[default_name(), kernel] * n
+    return None
 
 
 def cpu_baseline(warm_wl, cold_wl, atol, rtol, warm_every=1, cold_every=4, solver="rodas3"):
@@ -369,7 +378,7 @@ def bench_plain(args, solver="ros2"):
                    "flop_model_" + solver: {"per_cell_call": f_call, "per_substep": f_sub, "per_attempt": f_att}},
         "roofline": {"bound": "fp64", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS,
-                     "traffic": block_traffic(kernel, att_main / K),
+                     "traffic": block_traffic(kernel, st.main_cells, att_main / K),
                      "kernel": kernel, "avg_ms": main_ms / K,
                      "algorithmic_bytes": (2 * mech.nspecies * 4 + 4 * 4 + mech.nr_photo * 8) * grid.ncell},
     }
@@ -693,7 +702,7 @@ def main():
     pk = block_kernel()
     plain = {"kernel": pk, "bound": "fp64", "unit": "TFLOP/s",
              "avg_ms": b_main_ms / K, "achieved": b_flops_main / (b_main_ms * 1e-3) / 1e12,
-             "peak": FP64_PEAK_TFLOPS, "traffic": block_traffic(pk, b_att_main / K),
+             "peak": FP64_PEAK_TFLOPS, "traffic": block_traffic(pk, st.main_cells, b_att_main / K),
              "algorithmic_bytes": 528 * grid.ncell}
     plain["frac"] = plain["achieved"] / plain["peak"]
     if sur is None:
@@ -706,11 +715,10 @@ def main():
         mlp_ms = sum(s.mlp_ms for s in sstats)
         fb_flops = sum(rodas3_flops(s.fallback_cells, s.fallback_cell_substeps, s.fallback_cell_attempts)
                        for s in sstats)
-        fb_att = sum(s.fallback_cell_attempts for s in sstats)
         fk = block_kernel()
         fallback = {"kernel": fk, "bound": "fp64", "unit": "TFLOP/s",
                     "avg_ms": fb_ms / K, "achieved": fb_flops / max(fb_ms * 1e-3, 1e-9) / 1e12,
-                    "peak": FP64_PEAK_TFLOPS, "traffic": block_traffic(fk, fb_att / K),
+                    "peak": FP64_PEAK_TFLOPS, "traffic": None,        # of a list launch: not measured
                     "algorithmic_bytes": 528 * sum(s.fallback_cells for s in sstats) / K}
         fallback["frac"] = fallback["achieved"] / fallback["peak"]
         mlp = {"kernel": "mlp_infer<256,4,8,2>", "bound": "mfma", "unit": "TFLOP/s",

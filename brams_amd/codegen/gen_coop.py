@@ -19,6 +19,11 @@ The last `dense` pivots, nearly a dense block, are eliminated by one wave
 dependent pivots costs a barrier each when it is spread over waves, and a few
 FMA latencies when it is not.  Their rows of the matrix are assembled, and
 eliminated by the other pivots, on the other waves.
+
+coop_rows.json says for each mechanism how many waves, how large the dense
+block, and which wave owns the row of each pivot.  RELACS_TUV's rows were found
+by simulated annealing on Layout.stats; the search is not part of the
+repository.  Where rows is null, default_rows deals them.
 """
 LDS_SLOTS = 320                  # 160 KB / (64 lanes x 8 bytes)
 DENSE_PARTS = 3                  # phases of the dense wave's elimination

@@ -13,15 +13,19 @@
 // sub-step loop, the step-size controller and the write-back.
 //
 // Bound: a block's attempt is a chain of phases between barriers, each as long
-// as its busiest wave; one workgroup fills a CU (153 KB of LDS, 256 registers
+// as its busiest wave; one workgroup fills a CU (159 KB of LDS, 256 registers
 // a lane at two waves per SIMD), so nothing overlaps another block's.
 // Measured on 1.6M cells of RELACS_TUV, one step at the reference's
-// tolerances (16.2 attempts a cell): 30.9 ms, 20.6 us a block's attempt, of
-// which a wave is busy for half (a wave's registers hold its rows of the
-// matrix with little to spare, so the reads of LDS run only a few operations
-// ahead).  The kernel it replaces kept one lane's whole state in registers and
-// scratch: it read and wrote 63 KB of spilled state a cell-attempt and took
-// 353 ms.
+// tolerances (16.3 attempts a cell): 30.8 ms, 20.6 us or 49 000 clocks a
+// block's attempt.  57 % of a wave's clocks are waits (barriers, LDS), 14 %
+// waits for issue, 17 % FP64 and other vector instructions.  The attempt
+// sweeps its straight-line code (385 KB for the eight waves) with 5 500
+// fetches, of which 1.4 % miss the instruction cache or join a miss.  The
+// generator's model (Layout.stats) gives 31 800 clocks; what the other 17 000
+// are is not known.  A lane spills up to 176 bytes, which the caches hold:
+// memory sees 1.3 KB a cell whatever the attempts.  The kernel it replaces
+// kept one lane's whole state in registers and scratch: it read and wrote
+// 63 KB of spilled state a cell-attempt and took 353 ms.
 //
 // Blocks of 65..127 cells (the first ones of a grid whose cell count is no
 // multiple of 64) run as two halves in turn inside each attempt, with their
