@@ -21,7 +21,7 @@
 // concentrations, production and loss) filled the register file at one wave
 // per SIMD, spilled, and waited on its own chains: 2.19 ms for 1.6M cells of
 // RELACS_TUV, itchim 75, where memory needs 0.25 ms.  Shared out, a wave has
-// 16 reactions and 6 species, and four waves fit a SIMD: 0.97 ms, with no
+// 16 reactions and 6 species, and four waves fit a SIMD: 1.01 ms, with no
 // register spilled.
 #include <hip/hip_runtime.h>
 
