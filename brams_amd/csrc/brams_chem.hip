@@ -1296,8 +1296,8 @@ int host_step(const brams_chem_args* a, int solver) {
   // a PARALLEL step with N_DYN_CHEM=1 writes the transported species' sc_t and
   // the others' sc_p (rodas3:713-798)
   for (int s = 0; s < MECH_NS; ++s) {
-    if (need_t) h.out.push_back({a->sc_t[s], o_t + s * fsz, fsz});
-    if (!need_t || !flags[s]) h.out.push_back({a->sc_p[s], o_p + s * fsz, fsz});
+    const bool tend = need_t && flags[s];
+    h.out.push_back({tend ? a->sc_t[s] : a->sc_p[s], (tend ? o_t : o_p) + s * fsz, fsz});
   }
   h.out.push_back({a->last_accepted_dt, o_dt, sizeof(double) * nob});
   hipStream_t st = nullptr;

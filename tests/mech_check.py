@@ -387,7 +387,7 @@ def gpu_scale_ros2():
     assert np.array_equal(gfail[ran] != 0, ofail[ran] != 0) and (rc > 0) == (orc > 0), (rc, orc)
     assert np.array_equal(gatt[ids], oatt[ids]) and np.array_equal(gsub[ids], osub[ids])
     assert worst <= max(1e-6, 4 * sens), (worst, sens)
-    say("GPU ROS2 200x200x40 (four waves per SIMD, relaxed state): attempts per sampled block = oracle, "
+    say("GPU ROS2 200x200x40 (relaxed state): attempts per sampled block = oracle, "
         "%d failed blocks on both sides, worst %.2g (oracle's one-ulp sensitivity %.2g), %.1f ms"
         % (int(np.count_nonzero(gfail)), worst, sens, st.kernel_ms))
 
